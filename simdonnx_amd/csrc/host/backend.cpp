@@ -2959,11 +2959,52 @@ bool profiler_tool_loaded() {
     return loaded;
 }
 
+// The kernels that move a graph's fp32 host windows (pinned and mapped: the device reads and writes them in
+// place) to and from the arena in its storage type (staging.hip).
+struct Staging {
+    void *in = nullptr, *out = nullptr;  // sox_stage_in_*, sox_stage_out_*
+    void* cvt = nullptr;                 // 16-bit -> fp32 on the device, in front of a copy-engine download
+
+    // Downloads above this go through the copy engine: 30 MB take 556 us from the kernel and 557 with the
+    // conversion and the copy, 70 MB 1288 and ~1265.
+    static constexpr int64_t kEngineBytes = 32ll << 20;
+    static bool engine(int64_t out_count) { return out_count * 4 > kEngineBytes; }
+    // fp32 device staging a graph needs: only the 16-bit outputs that the copy engine fetches
+    static int64_t stage_floats(const sox_graph& g, int64_t out_count) { return g.f16 && engine(out_count) ? out_count : 0; }
+
+    void bind(const sox_graph& g) {
+        const std::string ty = g.bf16 ? "bf16" : g.f16 ? "f16" : "f32";
+        in = g.be->fn("sox_stage_in_" + ty);
+        out = g.be->fn("sox_stage_out_" + ty);
+        if (g.f16) cvt = g.be->fn("sox_" + ty + "_to_f32");
+    }
+    static void launch(void* fn, const void* x, void* y, int64_t count, int64_t blocks, void* stream) {
+        if (count <= 0) return;
+        sox_cvt_args a{x, y, count};
+        const uint32_t grid[3] = {(uint32_t)blocks, 1, 1}, block[3] = {256, 1, 1};
+        check(sox_launch(fn, grid, block, 0, stream, &a, sizeof a), "staging");
+    }
+    void upload(const float* host, void* dst, int64_t count, void* stream) const {
+        launch(in, host, dst, count, std::min<int64_t>(64, (count + 2047) / 2048), stream);
+    }
+    void download(const void* src, float* host, int64_t count, void* stage, bool f16, void* stream) const {
+        if (!engine(count)) {
+            launch(out, src, host, count, std::min<int64_t>(256, (count + 4095) / 4096), stream);
+            return;
+        }
+        if (f16) {
+            launch(cvt, src, stage, count, count / 1024 + 1, stream);
+            src = stage;
+        }
+        check(sox_memcpy_d2h(host, src, (size_t)count * 4, stream), "output download");
+    }
+};
+
 }  // namespace
 
 // Device buffers shared by the sessions of one owner that run one at a time (VkBufferPool /
 // VkSessionBuffers, Backends/Vulkan/VkBatch.cs:6-25, VkSession.cs:10-55): the arena slab, the device
-// fp32 staging of the 16-bit conversions and the pinned fp32 input / output staging. They grow to the
+// fp32 staging of large 16-bit outputs and the pinned fp32 input / output staging. They grow to the
 // largest session (by half again each time, as Ensure); growing replaces a buffer and bumps the
 // generation, which makes the sessions created before it stale. The borrowing sessions enqueue on the
 // pool's one stream, so their runs never overlap on the device.
@@ -3044,11 +3085,10 @@ struct sox_session {
     std::vector<int64_t> in_count;
     float* out_host = nullptr;
     int64_t out_count = 0;
-    void* stage = nullptr;  // device fp32 staging for the fp16 conversions
+    void* stage = nullptr;  // device fp32 staging of a 16-bit output that the copy engine fetches, or null
     void* sync = nullptr;   // the graph's cross-workgroup counters: this session's own, also on a pool
     std::vector<std::vector<uint8_t>> kernargs;
-    void* cvt_in = nullptr;
-    void* cvt_out = nullptr;
+    Staging staging;
     bool replay = false;
     void* exec_full = nullptr;
     void* exec_disp = nullptr;
@@ -3069,33 +3109,12 @@ struct sox_session {
         return (uint8_t*)arena + (uint64_t)g->plan.buf_offset[pv.buf] * g->es;
     }
 
-    void cvt(void* fn, const void* x, void* y, int64_t count) {
-        sox_cvt_args a{x, y, count};
-        uint32_t grid[3] = {(uint32_t)std::max<int64_t>(1, (count / 4 + 255) / 256 + 1), 1, 1}, block[3] = {256, 1, 1};
-        check(sox_launch(fn, grid, block, 0, stream, &a, sizeof a), "staging conversion");
-    }
-
     void stage_in() {
-        for (size_t i = 0; i < g->plan.inputs.size(); i++) {
-            void* dst = value_ptr(g->plan.inputs[i]);
-            if (g->f16) {
-                check(sox_memcpy_h2d(stage, in_host[i], (size_t)in_count[i] * 4, stream), "input upload");
-                cvt(cvt_in, stage, dst, in_count[i]);
-            } else {
-                check(sox_memcpy_h2d(dst, in_host[i], (size_t)in_count[i] * 4, stream), "input upload");
-            }
-        }
+        for (size_t i = 0; i < g->plan.inputs.size(); i++)
+            staging.upload(in_host[i], value_ptr(g->plan.inputs[i]), in_count[i], stream);
     }
 
-    void stage_out() {
-        void* src = value_ptr(g->plan.output);
-        if (g->f16) {
-            cvt(cvt_out, src, stage, out_count);
-            check(sox_memcpy_d2h(out_host, stage, (size_t)out_count * 4, stream), "output download");
-        } else {
-            check(sox_memcpy_d2h(out_host, src, (size_t)out_count * 4, stream), "output download");
-        }
-    }
+    void stage_out() { staging.download(value_ptr(g->plan.output), out_host, out_count, stage, g->f16, stream); }
 
     void dispatch(size_t i) {
         current();
@@ -3466,17 +3485,16 @@ int session_create(sox_graph* graph, sox_buffer_pool* pool, sox_session** sessio
         if (pool && pool->be != graph->be) fail(SOX_E_INVALID, "buffer pool of another backend");
         s->g = graph;
         graph->refs++;
-        int64_t stage = 0, in_total = 0;
+        int64_t in_total = 0;
         std::vector<int64_t> in_off;
         for (int v : graph->plan.inputs) {
             const int64_t n = graph->V(v).count();
             in_off.push_back(in_total);
             in_total += (n + 15) & ~15ll;  // each input 64-byte aligned in the shared staging
             s->in_count.push_back(n);
-            stage = std::max(stage, n);
         }
         s->out_count = graph->V(graph->plan.output).count();
-        stage = std::max(stage, s->out_count);
+        const int64_t stage = Staging::stage_floats(*graph, s->out_count);
         if (pool) {
             pool->ensure(graph->arena_bytes(), (uint64_t)stage * 4, (uint64_t)in_total * 4, (uint64_t)s->out_count * 4);
             s->pool = pool;
@@ -3497,7 +3515,7 @@ int session_create(sox_graph* graph, sox_buffer_pool* pool, sox_session** sessio
                 s->in_host.push_back(h);
             }
             check(sox_host_alloc((void**)&s->out_host, (size_t)s->out_count * 4), "output staging");
-            check(sox_malloc(&s->stage, (size_t)stage * 4), "device staging");
+            if (stage) check(sox_malloc(&s->stage, (size_t)stage * 4), "device staging");
         }
         if (graph->sync_bytes) {  // zero once: every launch leaves its counters at 0
             check(sox_malloc(&s->sync, graph->sync_bytes), "counters");
@@ -3505,8 +3523,7 @@ int session_create(sox_graph* graph, sox_buffer_pool* pool, sox_session** sessio
             check(sox_memcpy_h2d(s->sync, zeros.data(), zeros.size(), s->stream), "counters");
             check(sox_stream_sync(s->stream), "counters");
         }
-        s->cvt_in = graph->be->fn(graph->bf16 ? "sox_f32_to_bf16" : "sox_f32_to_f16");
-        s->cvt_out = graph->be->fn(graph->bf16 ? "sox_bf16_to_f32" : "sox_f16_to_f32");
+        s->staging.bind(*graph);
         for (const Dispatch& d : graph->disp) {
             std::vector<uint8_t> ka = d.kernarg;
             for (const Patch& p : d.patches) {
@@ -3720,9 +3737,9 @@ struct sox_ctc {
     void* w = nullptr;     // fp16 [columns][ldw]
     void* bias = nullptr;  // fp32 [columns]
     std::mutex mu;         // the workspace below is shared by the calls on this object
-    void* work = nullptr;  // part + indices + probs + status
+    void* work = nullptr;  // the column ranges' partials
     uint64_t work_bytes = 0;
-    void* host = nullptr;  // pinned: indices, probs, status
+    void* host = nullptr;  // pinned and mapped: indices, probs, status
     uint64_t host_bytes = 0;
 
     bool finite = true;    // weights and bias: a non-finite one makes every row's logits non-finite
@@ -3885,13 +3902,12 @@ int sox_ctc_argmax(sox_ctc* c, sox_session* s, int32_t feature_value, int32_t ba
         const int64_t R = L.R;
         std::lock_guard<std::mutex> lk(c->mu);
         const uint64_t part_b = ((uint64_t)L.splits * R * 12 + 255) & ~255ull, out_b = ((uint64_t)R * 4 + 255) & ~255ull;
-        const uint64_t need = part_b + 2 * out_b + 256;
-        if (need > c->work_bytes) {
+        if (part_b > c->work_bytes) {
             if (c->work) sox_free(c->work);
             c->work = nullptr;
             c->work_bytes = 0;
-            check(sox_malloc(&c->work, need), "CtcProjection workspace");
-            c->work_bytes = need;
+            check(sox_malloc(&c->work, part_b), "CtcProjection workspace");
+            c->work_bytes = part_b;
         }
         const uint64_t host_need = 2 * out_b + 256;
         if (host_need > c->host_bytes) {
@@ -3901,17 +3917,11 @@ int sox_ctc_argmax(sox_ctc* c, sox_session* s, int32_t feature_value, int32_t ba
             check(sox_host_alloc(&c->host, host_need), "CtcProjection staging");
             c->host_bytes = host_need;
         }
-        uint8_t* wk = (uint8_t*)c->work;
-        float* part = (float*)wk;
-        int32_t* d_idx = (int32_t*)(wk + part_b);
-        float* d_prob = (float*)(wk + part_b + out_b);
-        int32_t* d_status = (int32_t*)(wk + part_b + 2 * out_b);
+        // the merge pass writes its rows' results and the status into the mapped host block itself: three
+        // copy-engine downloads behind it took ~25 us of a call
         uint8_t* h = (uint8_t*)c->host;
         int32_t* h_status = (int32_t*)(h + 2 * out_b);
-        ctc_enqueue(c, s, L, part, d_idx, d_prob, d_status);
-        check(sox_memcpy_d2h(h, d_idx, (size_t)R * 4, s->stream), "CtcProjection indices");
-        check(sox_memcpy_d2h(h + out_b, d_prob, (size_t)R * 4, s->stream), "CtcProjection probabilities");
-        check(sox_memcpy_d2h(h_status, d_status, 4, s->stream), "CtcProjection status");
+        ctc_enqueue(c, s, L, (float*)c->work, (int32_t*)h, (float*)(h + out_b), h_status);
         check(sox_stream_sync(s->stream), "CtcProjection sync");
         if (*h_status) fail(SOX_E_INVALID, "Recognizer output is invalid.");
         memcpy(indices, h, (size_t)R * 4);
@@ -4067,11 +4077,12 @@ int sox_image_session_run(sox_image_session* is, sox_graph* graph, const uint8_t
 struct sox_unit_runner {
     struct Unit {
         sox_graph* g = nullptr;
-        uint64_t arena_off = 0, stage_off = 0;  // bytes into the shared device arena / device fp32 staging
+        uint64_t arena_off = 0, stage_off = 0;  // bytes into the shared device arena / download staging
         uint64_t sync_off = 0;                   // bytes into the shared counter block
         int64_t in_off = 0, out_off = 0;         // floats into the pinned host staging
         int64_t in_count = 0, out_count = 0;
         std::vector<std::vector<uint8_t>> kernargs;
+        Staging staging;
     };
     sox_backend* be = nullptr;
     std::vector<void*> streams;
@@ -4114,7 +4125,8 @@ struct sox_unit_runner {
             u.in_count = u.g->V(u.g->plan.inputs[0]).count();
             u.out_count = u.g->V(u.g->plan.output).count();
             u.stage_off = d;
-            d += ((uint64_t)std::max(u.in_count, u.out_count) * 4 + 255) & ~255ull;
+            d += ((uint64_t)Staging::stage_floats(*u.g, u.out_count) * 4 + 255) & ~255ull;
+            u.staging.bind(*u.g);
             u.in_off = hi;
             hi += (u.in_count + 63) & ~63ll;
             u.out_off = ho;
@@ -4137,7 +4149,7 @@ struct sox_unit_runner {
             have = need + need / 4;
         };
         grow_dev(arena, arena_bytes, std::max<uint64_t>(a, 256), "UnitRunner arena");
-        grow_dev(dstage, dstage_bytes, std::max<uint64_t>(d, 256), "UnitRunner staging");
+        grow_dev(dstage, dstage_bytes, d, "UnitRunner staging");
         if (sy > sync_bytes) {  // counters: zeroed when (re)allocated, back at 0 after every launch
             grow_dev(sync, sync_bytes, sy, "UnitRunner counters");
             std::vector<uint8_t> zeros(sync_bytes, 0);
@@ -4166,31 +4178,14 @@ struct sox_unit_runner {
         const PlanValue& pv = u.g->V(v);
         return (uint8_t*)arena + u.arena_off + (uint64_t)u.g->plan.buf_offset[pv.buf] * u.g->es;
     }
-    void cvt(void* fn, void* st, const void* x, void* y, int64_t count) {
-        sox_cvt_args a{x, y, count};
-        uint32_t grid[3] = {(uint32_t)std::max<int64_t>(1, (count / 4 + 255) / 256 + 1), 1, 1}, block[3] = {256, 1, 1};
-        check(sox_launch(fn, grid, block, 0, st, &a, sizeof a), "UnitRunner staging conversion");
-    }
     void run_unit(Unit& u, void* st) {
-        void* in = value_ptr(u, u.g->plan.inputs[0]);
-        void* out = value_ptr(u, u.g->plan.output);
-        void* ds = (uint8_t*)dstage + u.stage_off;
-        if (u.g->f16) {
-            check(sox_memcpy_h2d(ds, h_in + u.in_off, (size_t)u.in_count * 4, st), "UnitRunner upload");
-            cvt(be->fn(u.g->bf16 ? "sox_f32_to_bf16" : "sox_f32_to_f16"), st, ds, in, u.in_count);
-        } else {
-            check(sox_memcpy_h2d(in, h_in + u.in_off, (size_t)u.in_count * 4, st), "UnitRunner upload");
-        }
+        u.staging.upload(h_in + u.in_off, value_ptr(u, u.g->plan.inputs[0]), u.in_count, st);
         for (size_t i = 0; i < u.g->disp.size(); i++) {
             const Dispatch& d = u.g->disp[i];
             check(sox_launch(d.fn, d.grid, d.block, d.lds, st, u.kernargs[i].data(), u.kernargs[i].size()), d.name.c_str());
         }
-        if (u.g->f16) {
-            cvt(be->fn(u.g->bf16 ? "sox_bf16_to_f32" : "sox_f16_to_f32"), st, out, ds, u.out_count);
-            check(sox_memcpy_d2h(h_out + u.out_off, ds, (size_t)u.out_count * 4, st), "UnitRunner download");
-        } else {
-            check(sox_memcpy_d2h(h_out + u.out_off, out, (size_t)u.out_count * 4, st), "UnitRunner download");
-        }
+        u.staging.download(value_ptr(u, u.g->plan.output), h_out + u.out_off, u.out_count, dstage ? (uint8_t*)dstage + u.stage_off : nullptr,
+                           u.g->f16, st);
     }
 };
 

@@ -99,7 +99,7 @@ uint64_t sox_alloc_count(void) { return g_allocs.load(); }
 int sox_free(void* ptr) { return ptr ? st(hipFree(ptr)) : SOX_OK; }
 int sox_host_alloc(void** ptr, size_t bytes) {
     g_allocs++;
-    return st(hipHostMalloc(ptr, bytes ? bytes : 64, hipHostMallocDefault));
+    return st(hipHostMalloc(ptr, bytes ? bytes : 64, hipHostMallocCoherent | hipHostMallocMapped));
 }
 int sox_host_free(void* ptr) { return ptr ? st(hipHostFree(ptr)) : SOX_OK; }
 

@@ -1183,23 +1183,9 @@ extern "C" __global__ void __launch_bounds__(256) sox_slice_f32_v(sox_slice_copy
 extern "C" __global__ void __launch_bounds__(256) sox_slice_f32_s(sox_slice_copy_args p) { slice_body<float, 1>(p); }
 
 // ------------------------------------------------------------------------------------------
-// Staging conversions (f32to16.comp / f16to32.comp): fp16 / bf16 round to nearest even, as the
-// (Half) cast.
+// Output conversion of a download large enough for the copy engine (f16to32.comp); the others are
+// staging.hip's.
 // ------------------------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ void f32_to_body(const sox_cvt_args& p) {
-    typedef vec_t<T, 4> T4;
-    const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    const float* x = (const float*)p.x;
-    T* y = (T*)p.y;
-    if (i + 4 <= p.count) {
-        const float4v v = *(const float4v*)(x + i);
-        *(T4*)(y + i) = __builtin_convertvector(v, T4);  // round to nearest even
-    } else {
-        for (long j = i; j < p.count; j++) y[j] = (T)x[j];
-    }
-}
-
 template <typename T>
 __device__ __forceinline__ void to_f32_body(const sox_cvt_args& p) {
     typedef vec_t<T, 4> T4;
@@ -1214,8 +1200,6 @@ __device__ __forceinline__ void to_f32_body(const sox_cvt_args& p) {
     }
 }
 
-extern "C" __global__ void __launch_bounds__(256) sox_f32_to_f16(sox_cvt_args p) { f32_to_body<half_t>(p); }
-extern "C" __global__ void __launch_bounds__(256) sox_f32_to_bf16(sox_cvt_args p) { f32_to_body<bf16_t>(p); }
 extern "C" __global__ void __launch_bounds__(256) sox_f16_to_f32(sox_cvt_args p) { to_f32_body<half_t>(p); }
 extern "C" __global__ void __launch_bounds__(256) sox_bf16_to_f32(sox_cvt_args p) { to_f32_body<bf16_t>(p); }
 
