@@ -715,6 +715,96 @@ struct Emitter {
             (uint32_t)(tm * tn), 1, 1, 256, 0, label);
     }
 
+    // A tiling of the LDS-DMA ring and what it takes on MI355X, in us: with q tiles on the busiest CU and nk
+    // slices of bk, base + q tile + nk max(lat, q thr). lat is a slice's DMA and barrier round trip when the
+    // CU has one tile, thr a slice's share when several workgroups overlap theirs. The constants are fits to
+    // sweeps of every tiling over ~30 products (47 x 192 -> 768 to 8192 x 768 -> 3072) and ~20 convs; the
+    // estimates fall within ~15% of the measured times, and the pick within ~8% of the fastest tiling. The
+    // rule before, the largest tile that fills every resident slot, measured against the estimate's pick:
+    // Gemm 6000 x 320 -> 1280 19.9 / 11.9 us, 3000 x 3072 -> 768 51.0 / 34, 3000 x 768 -> 768 17.5 / 10.7,
+    // 1024 x 256 -> 3000 10.5 / 6.8, 786 x 768 -> 760 8.2 / 6.8; conv 8x64x64 128 -> 256 3x3 41.6 / 32.5,
+    // 2x95x127 96 -> 168 32.0 / 25.0, 2x160x160 40 -> 80 24.3 / 16.5, 1x80x80 64 -> 24 5x5 19.0 / 14.9.
+    struct RingCfg {
+        const char* name;
+        int bm, bn, bk, wgs_per_cu;
+        float lat, thr, base, tile;
+        int64_t tiles(int64_t m, int64_t n) const { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
+        uint32_t threads() const { return strstr(name, "_w8") ? 512 : 256; }
+    };
+    uint32_t ring_grid(const RingCfg& c, int64_t m, int64_t n) const {
+        const int64_t cus = std::max(1, g.be->info.compute_units);
+        return (uint32_t)std::min<int64_t>(c.tiles(m, n), cus * c.wgs_per_cu);
+    }
+    // The tiling of an m x n product over `taps` taps of k reduction elements each: the forced one, else the
+    // one of [first, last) with the smallest estimate
+    const RingCfg& ring_pick(const RingCfg* cfgs, size_t ncfg, int first, int last, int64_t m, int64_t n, int64_t k, int64_t taps,
+                             const char* forced, const char* what) const {
+        if (forced && *forced) {
+            for (size_t i = 0; i < ncfg; i++)
+                if (!strcmp(cfgs[i].name, forced)) return cfgs[i];
+            fail(SOX_E_INVALID, std::string(what) + ": unknown kernel " + forced);
+        }
+        const int64_t cus = std::max(1, g.be->info.compute_units);
+        int pick = first;
+        float best = 0.0f;
+        for (int i = first; i < last; i++) {
+            const RingCfg& c = cfgs[i];
+            const float q = (float)((c.tiles(m, n) + cus - 1) / cus), nk = (float)(taps * ((k + c.bk - 1) / c.bk));
+            const float t = c.base + q * c.tile + nk * std::max(c.lat, q * c.thr);
+            if (i == first || t < best) {
+                pick = i;
+                best = t;
+            }
+        }
+        return cfgs[pick];
+    }
+
+    // Dense product on the LDS-DMA ring (gemm_ring.h): a Gemm, or a 1x1 conv over its pixels. a holds m, n, k
+    // (a multiple of 8), ldy and the epilogue flags.
+    void launch_gemm_dma(int node, sox_igemm_args a, sox_bind x, sox_bind w, sox_bind bias, sox_bind add_b, sox_bind y,
+                         const sox_graph::LnFold* ln, const std::string& label) {
+        static const RingCfg cfgs16[] = {
+            {"sox_gemm_f16_256x192_w8k64s2", 256, 192, 64, 1, 1.6f, 1.6f, 4.0f, 2.0f},
+            {"sox_gemm_f16_256x128_w8k64s2", 256, 128, 64, 1, 1.3f, 1.3f, 3.3f, 2.0f},
+            {"sox_gemm_f16_128x128_k64s2", 128, 128, 64, 2, 0.72f, 0.67f, 4.0f, 1.6f},
+            {"sox_gemm_f16_128x64_k64s2e", 128, 64, 64, 2, 0.46f, 0.345f, 3.9f, 0.4f},
+            {"sox_gemm_f16_64x64_k64s2", 64, 64, 64, 4, 0.256f, 0.22f, 3.5f, 0.35f},
+            // selectable with SIMDONNX_HIP_GEMM (tuning / tests)
+            {"sox_gemm_f16_128x64_k64s2", 128, 64, 64, 3},     {"sox_gemm_f16_64x64_k64s4", 64, 64, 64, 2},
+            {"sox_gemm_f16_128x64_k64s4", 128, 64, 64, 1},     {"sox_gemm_f16_256x192_k32s5", 256, 192, 32, 1},
+            {"sox_gemm_f16_256x192_k32s4", 256, 192, 32, 1},   {"sox_gemm_f16_256x256_w8k32s4", 256, 256, 32, 1},
+            {"sox_gemm_f16_256x256_w8k64s2", 256, 256, 64, 1}, {"sox_gemm_f16_256x128_k32s3", 256, 128, 32, 2},
+            {"sox_gemm_f16_256x128_k32s5", 256, 128, 32, 1},   {"sox_gemm_f16_128x128_k32s4", 128, 128, 32, 2},
+            {"sox_gemm_f16_128x192_k32s3", 128, 192, 32, 2}};
+        // a K that is no multiple of 64 (a multiple of 8): 32-deep slices beside the 64-deep ones
+        static const RingCfg cfgs_kt[] = {
+            {"sox_gemm_kt_f16_256x128_w8k64s2", 256, 128, 64, 1, 1.3f, 1.3f, 3.3f, 2.0f},
+            {"sox_gemm_kt_f16_128x128_k64s2", 128, 128, 64, 2, 0.72f, 0.67f, 4.0f, 1.6f},
+            {"sox_gemm_kt_f16_128x64_k64s2", 128, 64, 64, 3, 0.5f, 0.42f, 3.9f, 0.5f},
+            {"sox_gemm_kt_f16_64x64_k64s2", 64, 64, 64, 4, 0.3f, 0.25f, 3.5f, 0.35f},
+            {"sox_gemm_kt_f16_128x96_k32s2", 128, 96, 32, 3, 0.3f, 0.26f, 4.0f, 0.7f},
+            {"sox_gemm_kt_f16_64x64_k32s2", 64, 64, 32, 4, 0.19f, 0.16f, 3.4f, 0.35f}};
+        const char* forced = getenv("SIMDONNX_HIP_GEMM");
+        const RingCfg* pick;
+        if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 6, 0, 6, a.m, a.n, a.k, 1, nullptr, "");
+        else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5, a.m, a.n, a.k, 1, forced, "SIMDONNX_HIP_GEMM");
+        a.kpad = pad8(a.k);
+        a.lda = a.k;
+        a.flags |= SOX_F_DENSE_A;
+        a.tiles_n = (a.n + pick->bn - 1) / pick->bn;
+        std::string kname = pick->name;
+        std::vector<std::pair<size_t, sox_bind>> ptrs = {
+            {offsetof(sox_igemm_args, x), x}, {offsetof(sox_igemm_args, w), w}, {offsetof(sox_igemm_args, bias), bias},
+            {offsetof(sox_igemm_args, add), add_b}, {offsetof(sox_igemm_args, y), y}, {offsetof(sox_igemm_args, zeros), none()}};
+        if (ln) {
+            kname = "sox_gemm_ln_f16_" + kname.substr(strlen("sox_gemm_f16_"));
+            if (kname.back() == 'e') kname.pop_back();  // (the folded 128x64 stores from registers)
+            a.ln_eps = ln->eps;
+            ptrs.push_back({offsetof(sox_igemm_args, ln_c), bind(ln->colsum, SOX_CK_F32)});
+        }
+        add(node, kname, a, ptrs, ring_grid(*pick, a.m, a.n), 1, 1, pick->threads(), 0, label);
+    }
+
     // Every window coordinate of a reflect-padded conv lies in [-(dim-1), 2 dim - 2], so one fold
     // maps it into the image (ONNX reflect pads are < dim; this also rejects 1-pixel axes).
     static bool reflect_folds_once(const sox_igemm_args& a) {
@@ -724,32 +814,25 @@ struct Emitter {
         return axis(a.ih, a.pt, a.sh, a.oh, a.kh) && axis(a.iw, a.pl, a.sw, a.ow, a.kw);
     }
 
-    // Implicit-GEMM conv on the LDS-DMA ring (gemm.hip, CONV mode): tile by output channels, 64-deep
-    // slices for long K, a persistent grid of two workgroups per CU at most.
-
+    // Implicit-GEMM conv on the LDS-DMA ring (gemm_ring.h, CONV mode): the large-conv tiles by rule, else the
+    // tiling with the smallest estimate.
     void launch_conv_dma(int node, sox_igemm_args a, sox_bind x, sox_bind w, sox_bind bias, sox_bind add_b,
                          sox_bind y) {
-        struct Cfg { const char* name; int bm, bn, wgs_per_cu; };
-        static const Cfg cfgs[] = {
-            {"sox_conv_f16_128x32_k32s4", 128, 32, 2},  {"sox_conv_f16_128x32_k64s6", 128, 32, 1},
-            {"sox_conv_f16_64x64_k32s4", 64, 64, 2},    {"sox_conv_f16_64x64_k64s4", 64, 64, 2},
-            {"sox_conv_f16_64x64_k64s8", 64, 64, 1},    {"sox_conv_f16_128x128_k32s4", 128, 128, 2},
-            {"sox_conv_f16_128x64_k32s4", 128, 64, 2},  {"sox_conv_f16_128x64_k64s3", 128, 64, 2},
-            {"sox_conv_f16_128x64_k64s5", 128, 64, 1},  {"sox_conv_f16_256x128_w8k64s2", 256, 128, 1},
-            {"sox_conv_f16_256x256_w8k64s2", 256, 256, 1}, {"sox_conv_f16_h256", 256, 256, 1}};
-        auto find = [&](const char* nm) -> const Cfg* {
-            for (const Cfg& c : cfgs)
-                if (!strcmp(c.name, nm)) return &c;
-            fail(SOX_E_INVALID, std::string("conv kernel ") + nm + " unknown");
-        };
+        static const RingCfg cfgs16[] = {
+            {"sox_conv_f16_128x128_k64s2", 128, 128, 64, 2, 1.0f, 0.72f, 4.5f, 1.2f},
+            {"sox_conv_f16_128x96_k64s2", 128, 96, 64, 2, 0.8f, 0.57f, 4.2f, 0.8f},
+            {"sox_conv_f16_128x96_k32s2", 128, 96, 32, 3, 0.5f, 0.365f, 4.2f, 0.8f},
+            {"sox_conv_f16_128x64_k64s2", 128, 64, 64, 3, 0.6f, 0.39f, 4.0f, 0.6f},
+            {"sox_conv_f16_64x64_k64s4", 64, 64, 64, 2, 0.42f, 0.29f, 3.8f, 0.4f},
+            {"sox_conv_f16_64x64_k32s4", 64, 64, 32, 2, 0.28f, 0.18f, 3.8f, 0.4f},
+            // by the rules for large convs below
+            {"sox_conv_f16_256x128_w8k64s2", 256, 128, 64, 1}, {"sox_conv_f16_256x256_w8k64s2", 256, 256, 64, 1},
+            {"sox_conv_f16_h256", 256, 256, 64, 1}};
         // the ring keeps each row's receptive-field origin in 16 bits a coordinate and W offsets in 32
         if (a.ih > 30000 || a.iw > 30000) unsupported("conv: an image side over 30000 pixels");
         if ((int64_t)a.n * a.kpad >= (int64_t)1 << 31) unsupported("conv: weights of 2^31 elements or more");
         const int64_t cus = std::max(1, g.be->info.compute_units);
         auto tiles = [&](int bm, int bn) { return ((a.m + bm - 1) / bm) * (int64_t)((a.n + bn - 1) / bn); };
-        // slices are channel blocks of one tap: 64-deep when that divides ic or ic > 96 (fewer slices
-        // outweigh a zero-filled half block there), else 32-deep; four stages, two workgroups per CU
-        const bool bk64 = a.ic % 64 == 0 || a.ic > 96, deep = a.k >= 512;
         // the input has fewer than 2^31 elements (the 256x256 tile's 32-bit DMA offsets); m = n * oh * ow
         // (a ConvTranspose's A side is its input pixels: oh, ow = ih, iw)
         const bool in32 = (int64_t)(a.m / ((int64_t)a.oh * a.ow)) * a.ih * a.iw * a.ic < ((int64_t)1 << 31);
@@ -760,7 +843,7 @@ struct Emitter {
         const bool h256_ok = a.kh == 3 && a.kw == 3 && a.sh == 1 && a.sw == 1 && a.pt == 1 && a.pl == 1 &&
                              a.oh == a.ih && a.ow == a.iw && a.ic % 64 == 0 && a.n % 256 == 0 &&
                              !(a.flags & (SOX_F_REFLECT | SOX_F_CONVT | SOX_F_DENSE_A)) && a.res_shift == 0;
-        const char* name;
+        const char* name = nullptr;
         const char* forced = getenv("SIMDONNX_HIP_CONV");  // tuning / tests
         if (forced && *forced) name = forced;
         else if (h256_ok && h256_tiles >= 2 * cus && !getenv("SIMDONNX_HIP_NO_H256"))
@@ -775,12 +858,8 @@ struct Emitter {
                  tiles(256, 128) >= 2 * cus)
             // large convs: at least two rounds of 256x128 tiles on every CU, 8 waves each
             name = "sox_conv_f16_256x128_w8k64s2";
-        else if (a.n <= 32) name = bk64 && deep ? "sox_conv_f16_128x32_k64s6" : "sox_conv_f16_128x32_k32s4";
-        else if (a.n <= 64 || (tiles(128, 128) < cus && tiles(128, 64) < cus))
-            name = bk64 ? "sox_conv_f16_64x64_k64s4" : "sox_conv_f16_64x64_k32s4";
-        else if (tiles(128, 128) >= cus) name = "sox_conv_f16_128x128_k32s4";
-        else name = bk64 ? "sox_conv_f16_128x64_k64s3" : "sox_conv_f16_128x64_k32s4";
-        const Cfg* c = find(name);
+        const int64_t taps = (int64_t)a.kh * a.kw;
+        const RingCfg* c = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV");
         if (!in32 && !strcmp(c->name, "sox_conv_f16_256x256_w8k64s2"))
             unsupported("conv: the 256x256 tile takes inputs of fewer than 2^31 elements");
         if (!strcmp(c->name, "sox_conv_f16_h256")) {
@@ -798,8 +877,7 @@ struct Emitter {
             {{offsetof(sox_igemm_args, x), x}, {offsetof(sox_igemm_args, w), w}, {offsetof(sox_igemm_args, bias), bias},
              {offsetof(sox_igemm_args, add), add_b}, {offsetof(sox_igemm_args, y), y},
              {offsetof(sox_igemm_args, zeros), none()}},
-            (uint32_t)std::min<int64_t>(tiles(c->bm, c->bn), cus * c->wgs_per_cu), 1, 1,
-            strstr(c->name, "_w8") ? 512 : 256, 0, "conv");
+            ring_grid(*c, a.m, a.n), 1, 1, c->threads(), 0, "conv");
     }
 
     // a conv emitted in another node's place (plan_upsample_add): its output, and a residual read as the
@@ -1031,6 +1109,14 @@ struct Emitter {
                    (p.pad_mode != 1 || reflect_folds_once(a)) && !getenv("SIMDONNX_HIP_IGEMM")) {
             // fp16 NHWC with ic % 8 == 0 and zero/reflect padding: the LDS-DMA implicit-GEMM ring
             a.res_shift = cov.shift;
+            const char* forced = getenv("SIMDONNX_HIP_CONV");
+            if (kh == 1 && kw == 1 && st == 1 && p.strides[1] == 1 && !p.pads[0] && !p.pads[1] && !p.pads[2] &&
+                !p.pads[3] && cov.res < 0 && ih <= 30000 && iw <= 30000 && (int64_t)oc * a.kpad < ((int64_t)1 << 31) &&
+                !(forced && *forced)) {
+                // a 1x1 conv over its pixels is a dense product: no receptive fields to address
+                launch_gemm_dma(ni, a, xb, wb, p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(),
+                                p.add_value >= 0 ? bind(p.add_value) : none(), ybind, nullptr, "conv");
+            } else
             launch_conv_dma(ni, a, xb, wb,
                             p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(),
                             cov.res >= 0 ? bind(cov.res) : p.add_value >= 0 ? bind(p.add_value) : none(), ybind);
@@ -1183,13 +1269,13 @@ struct Emitter {
         const sox_bind res_b = residual >= 0 ? bind(residual) : none();
         a.flags = (p.bias_value >= 0 ? SOX_F_BIAS : 0) | (act << SOX_F_ACT_SHIFT) | (residual >= 0 ? SOX_F_RESIDUAL : 0);
         a.ldy = nn;
-        // large fp16 Gemms: the LDS-DMA pipelined persistent kernel (K in 64-slices, N in 4-channel groups;
-        // other N keep 8-byte-aligned rows only through the implicit-GEMM kernel's element stores)
+        // rows of whole 16-byte chunks: the LDS-DMA pipelined persistent kernel (any N: rows that are not
+        // whole 4-element groups are stored element by element)
         auto pad_it = g.padded_ld.find(out_value);
         const bool pad_rows = pad_it != g.padded_ld.end();
         auto ln_it = g.ln_fold.find(ni);
         const bool ln = ln_it != g.ln_fold.end();  // A is a folded LayerNorm's input
-        const bool dma = g.f16 && k % 64 == 0 && (nn % 4 == 0 || pad_rows) && m >= 64;
+        const bool dma = g.f16 && k % ld() == 0;
         if (ln && !dma) fail(SOX_E_INVALID, "Gemm: LayerNorm folded into a Gemm off the LDS-DMA route");
         // opt-in (SIMDONNX_HIP_GEMMPP): whole 256 x 128 tiles, K = 768, bias + none / relu / GELU, at
         // least a tile per CU, on the kernel that runs each tile's epilogue under the next tile's
@@ -1218,56 +1304,14 @@ struct Emitter {
             return;
         }
         if (dma) {
-            struct Cfg { const char* name; int bm, bn, threads, wgs_per_cu; };
-            static const Cfg cfgs[] = {
-                // defaults, largest first: the first whose tile count fills every resident slot
-                {"sox_gemm_f16_256x192_w8k64s2", 256, 192, 512, 1}, {"sox_gemm_f16_256x128_w8k64s2", 256, 128, 512, 1},
-                {"sox_gemm_f16_128x128_k64s2", 128, 128, 256, 2},   {"sox_gemm_f16_128x64_k64s2", 128, 64, 256, 3},
-                {"sox_gemm_f16_64x64_k64s4", 64, 64, 256, 2},
-                // selectable with SIMDONNX_HIP_GEMM (tuning / tests)
-                {"sox_gemm_f16_64x64_k64s2", 64, 64, 256, 4},       {"sox_gemm_f16_128x64_k64s4", 128, 64, 256, 1},
-                {"sox_gemm_f16_256x192_k32s5", 256, 192, 256, 1},   {"sox_gemm_f16_256x192_k32s4", 256, 192, 256, 1},
-                {"sox_gemm_f16_256x256_w8k32s4", 256, 256, 512, 1}, {"sox_gemm_f16_256x256_w8k64s2", 256, 256, 512, 1},
-                {"sox_gemm_f16_256x128_k32s3", 256, 128, 256, 2},   {"sox_gemm_f16_256x128_k32s5", 256, 128, 256, 1},
-                {"sox_gemm_f16_128x128_k32s4", 128, 128, 256, 2}, {"sox_gemm_f16_128x192_k32s3", 128, 192, 256, 2}};
-            const int ncfg = (int)(sizeof(cfgs) / sizeof(cfgs[0]));
-            const char* forced = getenv("SIMDONNX_HIP_GEMM");
-            const Cfg* pick = nullptr;
-            if (forced && *forced) {
-                for (int i = 0; i < ncfg; i++)
-                    if (!strcmp(cfgs[i].name, forced)) pick = &cfgs[i];
-                if (!pick) fail(SOX_E_INVALID, std::string("SIMDONNX_HIP_GEMM: unknown kernel ") + forced);
-            } else {
-                // the largest of the default tilings that still gives every resident workgroup a tile
-                // (the LayerNorm-folded kernels exist for the four smaller ones)
-                const int cus = std::max(1, g.be->info.compute_units);
-                for (int i = ln ? 1 : 0; i < 5; i++) {
-                    pick = &cfgs[i];
-                    int64_t t = ((m + cfgs[i].bm - 1) / cfgs[i].bm) * ((nn + cfgs[i].bn - 1) / cfgs[i].bn);
-                    if (t >= (int64_t)cus * cfgs[i].wgs_per_cu) break;
-                }
-            }
             sox_igemm_args a{};
-            a.m = (int)m; a.n = nn; a.k = k; a.kpad = pad8(k);
-            a.flags = (p.bias_value >= 0 ? SOX_F_BIAS : 0) | (act << SOX_F_ACT_SHIFT) | SOX_F_DENSE_A |
+            a.m = (int)m; a.n = nn; a.k = k;
+            a.flags = (p.bias_value >= 0 ? SOX_F_BIAS : 0) | (act << SOX_F_ACT_SHIFT) |
                       (residual >= 0 ? SOX_F_RESIDUAL : 0) | (pad_rows ? SOX_F_PAD_ROWS : 0);
-            a.ldy = pad_rows ? pad_it->second : nn; a.lda = k;
-            a.tiles_n = (nn + pick->bn - 1) / pick->bn;
-            int64_t tiles = ((m + pick->bm - 1) / pick->bm) * (int64_t)a.tiles_n;
-            int64_t resident = (int64_t)std::max(1, g.be->info.compute_units) * pick->wgs_per_cu;
-            std::string kname = pick->name;
-            std::vector<std::pair<size_t, sox_bind>> ptrs = {
-                {offsetof(sox_igemm_args, x), bind(n.in[0])},
-                {offsetof(sox_igemm_args, w), bind(n.in[1], p.trans_b ? CK_GEMMNK_T : SOX_CK_GEMMNK)},
-                {offsetof(sox_igemm_args, bias), p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none()},
-                {offsetof(sox_igemm_args, add), res_b}, {offsetof(sox_igemm_args, y), bind(out_value)}};
-            if (ln) {
-                kname = "sox_gemm_ln_f16_" + kname.substr(strlen("sox_gemm_f16_"));
-                a.ln_eps = ln_it->second.eps;
-                ptrs.push_back({offsetof(sox_igemm_args, ln_c), bind(ln_it->second.colsum, SOX_CK_F32)});
-            }
-            add(ni, kname, a, ptrs, (uint32_t)std::min(tiles, resident), 1, 1, (uint32_t)pick->threads, 0,
-                ln ? "gemm_ln" : "gemm");
+            a.ldy = pad_rows ? pad_it->second : nn;
+            launch_gemm_dma(ni, a, bind(n.in[0]), bind(n.in[1], p.trans_b ? CK_GEMMNK_T : SOX_CK_GEMMNK),
+                            p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(), res_b, bind(out_value),
+                            ln ? &ln_it->second : nullptr, ln ? "gemm_ln" : "gemm");
             return;
         }
         char amode;
@@ -2260,7 +2304,7 @@ void plan_padded_rows(sox_graph& g) {
         const PlanValue& av = P.values[n.in[0]];
         const int N = yv.shape.back(), K = av.shape.back();
         if (N % 4 == 0 || K % 64 != 0 || yv.buf < 0 || y == P.output || yv.phys().back() != N) continue;
-        if (av.count() / K < 64 || value_reads(g, y) != 1) continue;
+        if (value_reads(g, y) != 1) continue;
         bool viewed = false;  // a view of y would read the unpadded layout
         for (int v = 0; v < (int)P.values.size() && !viewed; v++) viewed = v != y && P.values[v].buf == yv.buf;
         if (viewed) continue;
@@ -2382,6 +2426,9 @@ void plan_convt_chain(sox_graph& g) {
     }
 }
 
+int fusable_attention(sox_graph& g, int qi, int x);
+bool fusable_mlp(sox_graph& g, int f1, int x, sox_graph::Mlp& f);
+
 // A LayerNorm over the innermost dim whose output only an fp16 Gemm reads, as its A (the recognizer
 // blocks' ln1 -> qkv and ln2 -> fc1, the final norm -> head): the LayerNorm folds into the Gemm,
 // which then reads the LayerNorm's input and normalises its rows itself (sox_gemm_ln_* kernels):
@@ -2390,8 +2437,8 @@ void plan_convt_chain(sox_graph& g) {
 // rounded to fp16 (the values the kernel multiplies) as ln_c. The mean and variance come from one
 // pass of sums and sums of squares, as the reference's GPU LayerNorm takes them
 // (Backends/Vulkan/Shaders/layernorm.comp:24-38). Taken only where the Gemm runs on the LDS-DMA
-// ring (K % 64 == 0, >= 64 rows, N % 4 == 0 or padded rows) and no node in between writes over
-// the LayerNorm's input; the Gemm's output moves to a buffer of its own when the arena plan put it
+// ring (K % 64 == 0, N % 4 == 0 or padded rows; at least 64 rows, or fewer where the Gemm then runs in
+// a fused attention or MLP) and no node in between writes over the LayerNorm's input; the Gemm's output moves to a buffer of its own when the arena plan put it
 // over that input (dead after the LayerNorm, read by the Gemm now).
 void fold_layernorm_into_gemm(sox_graph& g) {
     if (!g.f16 || getenv("SIMDONNX_HIP_NO_LN_FOLD")) return;
@@ -2406,7 +2453,7 @@ void fold_layernorm_into_gemm(sox_graph& g) {
         const float eps = ln.p<sox_ln_p>().eps;
         const PlanValue &xv = P.values[x], &gv = P.values[ln.in[1]], &bv = P.values[ln.in[2]];
         const int K = xv.shape.back();
-        if (xv.buf < 0 || xv.phys().back() != K || K % 64 != 0 || xv.count() / K < 64) continue;
+        if (xv.buf < 0 || xv.phys().back() != K || K % 64 != 0) continue;
         if (!gv.is_const || !bv.is_const || (int)gv.floats.size() != K || (int)bv.floats.size() != K) continue;
         if (y == P.output || value_reads(g, y) != 1) continue;
         int gi = -1;
@@ -2430,6 +2477,7 @@ void fold_layernorm_into_gemm(sox_graph& g) {
             if (!g.folded.count(k))
                 for (int o : P.nodes[k].out) clobbered |= overlap(value_range(P, o), xr);
         if (clobbered) continue;
+        if (xv.count() / K < 64) continue;
         PlanValue w2 = wv, b2, c2;
         w2.name = wv.name + ".ln";
         std::vector<double> bsum(N, 0.0), csum(N, 0.0);
@@ -2472,48 +2520,52 @@ void fold_layernorm_into_gemm(sox_graph& g) {
 // own rows of x and of the residual before it writes the same rows of the output, so the output may
 // share x's or the residual's buffer only at the same offset with the same row length; otherwise it
 // moves to a buffer of its own.
+// Whether f1, the Gemm that folds a LayerNorm of x, and the Gemm after it are such an MLP (f: its parts).
+bool fusable_mlp(sox_graph& g, int f1, int x, sox_graph::Mlp& f) {
+    if (!g.f16 || getenv("SIMDONNX_HIP_NO_MLP_FUSE") || g.folded.count(f1)) return false;
+    auto& P = g.plan;
+    const PlanNode& n1 = P.nodes[f1];
+    const sox_gemm_p p1 = n1.p<sox_gemm_p>();
+    if (p1.act != SOX_ACT_GELU || p1.trans_b) return false;
+    const int h = n1.out[0];
+    const int K1 = P.values[x].shape.back(), H = P.values[h].shape.back();
+    if (!((K1 == 192 && H == 768) || (K1 == 128 && H == 512) || (K1 == 64 && H == 256))) return false;
+    if (h == P.output || value_reads(g, h) != 1 || g.padded_ld.count(h)) return false;
+    int f2 = -1;
+    for (int k = f1 + 1; k < (int)P.nodes.size() && f2 < 0; k++)
+        if (!g.folded.count(k))
+            for (int v : P.nodes[k].in)
+                if (v == h) f2 = k;
+    if (f2 < 0 || g.ln_fold.count(f2)) return false;
+    // the kernel runs at f1's place: nothing may run between the two Gemms (it would see the output
+    // early), and the residual must exist by then
+    for (int k = f1 + 1; k < f2; k++)
+        if (!g.folded.count(k)) return false;
+    const PlanNode& n2 = P.nodes[f2];
+    if (n2.op != SOX_OP_GEMM || n2.in[0] != h || n2.in[1] == h) return false;
+    const sox_gemm_p p2 = n2.p<sox_gemm_p>();
+    const PlanValue& w2 = P.values[n2.in[1]];
+    if (p2.trans_b || p2.act != 0 || !w2.is_const || w2.shape.size() != 2 || w2.shape[0] != H) return false;
+    const int N2 = w2.shape[1];
+    if (N2 % 32 != 0 || N2 > 256) return false;
+    auto ra = g.residual_add.find(f2);
+    const int add = ra == g.residual_add.end() ? -1 : ra->second.first;
+    const int res = ra == g.residual_add.end() ? -1 : ra->second.second;
+    for (int k = f2 + 1; k < add; k++)  // the Add follows f2 directly (plan_residual_adds), nothing else
+        if (!g.folded.count(k)) return false;
+    const int out = add >= 0 ? P.nodes[add].out[0] : n2.out[0];
+    if (g.padded_ld.count(out) || P.values[out].shape.back() != N2) return false;
+    f = {f2, add, res, out};
+    return true;
+}
+
 void plan_fused_mlp(sox_graph& g) {
-    if (!g.f16 || getenv("SIMDONNX_HIP_NO_MLP_FUSE")) return;
     auto& P = g.plan;
     for (auto& kv : g.ln_fold) {
-        const int f1 = kv.first;
-        if (g.folded.count(f1)) continue;
-        const PlanNode& n1 = P.nodes[f1];
-        const sox_gemm_p p1 = n1.p<sox_gemm_p>();
-        if (p1.act != SOX_ACT_GELU || p1.trans_b || p1.bias_value < 0) continue;
-        const int h = n1.out[0];
-        const int K1 = P.values[n1.in[0]].shape.back(), H = P.values[h].shape.back();
-        if (!((K1 == 192 && H == 768) || (K1 == 128 && H == 512) || (K1 == 64 && H == 256))) continue;
-        if (h == P.output || value_reads(g, h) != 1 || g.padded_ld.count(h)) continue;
-        int f2 = -1;
-        for (int k = f1 + 1; k < (int)P.nodes.size() && f2 < 0; k++)
-            if (!g.folded.count(k))
-                for (int v : P.nodes[k].in)
-                    if (v == h) f2 = k;
-        if (f2 < 0 || g.ln_fold.count(f2)) continue;
-        // the kernel runs at f1's place: nothing may run between the two Gemms (it would see the output
-        // early), and the residual must exist by then
-        bool between = false;
-        for (int k = f1 + 1; k < f2; k++) between |= !g.folded.count(k);
-        if (between) continue;
-        const PlanNode& n2 = P.nodes[f2];
-        if (n2.op != SOX_OP_GEMM || n2.in[0] != h || n2.in[1] == h) continue;
-        const sox_gemm_p p2 = n2.p<sox_gemm_p>();
-        const PlanValue& w2 = P.values[n2.in[1]];
-        if (p2.trans_b || p2.act != 0 || !w2.is_const || w2.shape.size() != 2 || w2.shape[0] != H) continue;
-        const int N2 = w2.shape[1];
-        if (N2 % 32 != 0 || N2 > 256) continue;
-        auto ra = g.residual_add.find(f2);
-        const int add = ra == g.residual_add.end() ? -1 : ra->second.first;
-        const int res = ra == g.residual_add.end() ? -1 : ra->second.second;
-        if (add >= 0) {
-            bool between_add = false;  // the Add follows f2 directly (plan_residual_adds), nothing else
-            for (int k = f2 + 1; k < add; k++) between_add |= !g.folded.count(k);
-            if (between_add) continue;
-        }
-        const int out = add >= 0 ? P.nodes[add].out[0] : n2.out[0];
-        if (g.padded_ld.count(out) || P.values[out].shape.back() != N2) continue;
-        const int x = n1.in[0];
+        const int f1 = kv.first, x = P.nodes[f1].in[0];
+        sox_graph::Mlp f;
+        if (!fusable_mlp(g, f1, x, f) || P.nodes[f1].p<sox_gemm_p>().bias_value < 0) continue;
+        const int out = f.out, res = f.residual, K1 = P.values[x].shape.back(), N2 = P.values[out].shape.back();
         auto same_rows = [&](int v, int row_len) {
             return value_range(P, v).first == value_range(P, out).first && row_len == N2;
         };
@@ -2526,11 +2578,10 @@ void plan_fused_mlp(sox_graph& g) {
         // fc2 sums meet in sox_mlp_sum_*); SIMDONNX_HIP_MLP_SPLIT=0 / 1 forces either form
         const int64_t rbs = (P.values[x].count() / K1 + 31) / 32;
         const char* mode = getenv("SIMDONNX_HIP_MLP_SPLIT");
-        sox_graph::Mlp f{f2, add, res, out};
         f.split = mode && *mode ? mode[0] == '1' : rbs < std::max(1, g.be->info.compute_units);
         g.mlp[f1] = f;
-        g.folded.insert(f2);
-        if (add >= 0) g.folded.insert(add);
+        g.folded.insert(f.fc2);
+        if (f.add >= 0) g.folded.insert(f.add);
     }
 }
 
@@ -2540,51 +2591,55 @@ void plan_fused_mlp(sox_graph& g) {
 // t <= 96, the attention output is stored [n][t][heads][32] and nothing else reads the qkv rows (they
 // then stay in LDS). A workgroup reads its image's x rows while the image's other heads write their
 // output columns, so the output must not overlap x.
-void plan_fused_attention(sox_graph& g) {
-    if (!g.f16 || getenv("SIMDONNX_HIP_NO_ATTN_FUSE")) return;
+// fusable_attention: the Attention node that Gemm qi, which folds a LayerNorm of x, runs with, or -1.
+int fusable_attention(sox_graph& g, int qi, int x) {
+    if (!g.f16 || getenv("SIMDONNX_HIP_NO_ATTN_FUSE")) return -1;
     auto& P = g.plan;
-    const int nn = (int)P.nodes.size();
-    for (auto& kv : g.ln_fold) {
-        const int qi = kv.first, ai = qi + 1;
-        if (ai >= nn || g.folded.count(qi) || g.mlp.count(qi) || g.folded.count(ai)) continue;
-        const PlanNode &nq = P.nodes[qi], &na = P.nodes[ai];
-        if (na.op != SOX_OP_ATTENTION) continue;
-        const sox_gemm_p pq = nq.p<sox_gemm_p>();
-        if (pq.act != 0 || g.residual_add.count(qi)) continue;
-        const int x = nq.in[0], qkv = nq.out[0], att = na.out[0];
-        const PlanValue &xv = P.values[x], &qv = P.values[qkv], &ov = P.values[att];
-        constexpr int DIM = 192;
-        if (xv.buf < 0 || !xv.layout.empty() || xv.shape.back() != DIM || g.padded_ld.count(x)) continue;
-        if (qv.buf < 0 || !qv.layout.empty() || qv.shape.back() != 3 * DIM || g.padded_ld.count(qkv)) continue;
-        const int64_t rows = xv.count() / DIM;
-        // the attention reads q, k, v as [n][t][3][heads][32] views of the qkv rows, one image per n
-        const auto& pa = na.p<sox_attention_p>();
-        bool ok = true;
-        int64_t nb = -1, t = -1;
-        for (int i = 0; i < 3 && ok; i++) {
-            const PlanValue& v = P.values[na.in[i]];
-            const int* d = pa.dims[i];
-            ok = v.buf == qv.buf && v.count() == qv.count() && d[0] >= 0 && d[1] >= 0 && d[2] >= 0 &&
-                 pa.fix_axis[i] >= 0 && pa.fix_index[i] == i;
-            if (!ok) break;
-            if (i == 0) {
-                nb = v.shape[d[0]];
-                t = v.shape[d[2]];
-            }
-            ok = v.shape[d[0]] == nb && v.shape[d[1]] * 32 == DIM && v.shape[d[2]] == t && v.shape[d[3]] == 32 &&
-                 axis_stride(v, d[0]) == t * 3 * DIM && axis_stride(v, d[1]) == 32 &&
-                 axis_stride(v, d[2]) == 3 * DIM && axis_stride(v, d[3]) == 1 &&
-                 axis_stride(v, pa.fix_axis[i]) == DIM;
+    const int ai = qi + 1;
+    if (ai >= (int)P.nodes.size() || g.folded.count(qi) || g.mlp.count(qi) || g.folded.count(ai)) return -1;
+    const PlanNode &nq = P.nodes[qi], &na = P.nodes[ai];
+    if (na.op != SOX_OP_ATTENTION) return -1;
+    const sox_gemm_p pq = nq.p<sox_gemm_p>();
+    if (pq.act != 0 || g.residual_add.count(qi)) return -1;
+    const int qkv = nq.out[0], att = na.out[0];
+    const PlanValue &xv = P.values[x], &qv = P.values[qkv], &ov = P.values[att];
+    constexpr int DIM = 192;
+    if (xv.buf < 0 || !xv.layout.empty() || xv.shape.back() != DIM || g.padded_ld.count(x)) return -1;
+    if (qv.buf < 0 || !qv.layout.empty() || qv.shape.back() != 3 * DIM || g.padded_ld.count(qkv)) return -1;
+    const int64_t rows = xv.count() / DIM;
+    // the attention reads q, k, v as [n][t][3][heads][32] views of the qkv rows, one image per n
+    const auto& pa = na.p<sox_attention_p>();
+    int64_t nb = -1, t = -1;
+    for (int i = 0; i < 3; i++) {
+        const PlanValue& v = P.values[na.in[i]];
+        const int* d = pa.dims[i];
+        if (v.buf != qv.buf || v.count() != qv.count() || d[0] < 0 || d[1] < 0 || d[2] < 0 || pa.fix_axis[i] < 0 ||
+            pa.fix_index[i] != i)
+            return -1;
+        if (i == 0) {
+            nb = v.shape[d[0]];
+            t = v.shape[d[2]];
         }
-        if (!ok || nb * t != rows || t < 1 || t > 96) continue;
-        // output [n, h, t, d] stored as [n][t][h][d]
-        int ol[4] = {0, 1, 2, 3};
-        if (pa.out_layout[0] >= 0)
-            for (int i = 0; i < 4; i++) ol[i] = pa.out_layout[i];
-        if (!(ol[0] == 0 && ol[1] == 2 && ol[2] == 1 && ol[3] == 3) || ov.buf < 0 || ov.count() != rows * DIM) continue;
-        if (buffer_reads(g, qkv, ai) != 0) continue;
-        const auto xr = value_range(P, x), o = value_range(P, att);
-        if (xr.first < o.second && o.first < xr.second) continue;  // (views of the output share its buffer)
+        if (v.shape[d[0]] != nb || v.shape[d[1]] * 32 != DIM || v.shape[d[2]] != t || v.shape[d[3]] != 32 ||
+            axis_stride(v, d[0]) != t * 3 * DIM || axis_stride(v, d[1]) != 32 || axis_stride(v, d[2]) != 3 * DIM ||
+            axis_stride(v, d[3]) != 1 || axis_stride(v, pa.fix_axis[i]) != DIM)
+            return -1;
+    }
+    if (nb * t != rows || t < 1 || t > 96) return -1;
+    // output [n, h, t, d] stored as [n][t][h][d]
+    int ol[4] = {0, 1, 2, 3};
+    if (pa.out_layout[0] >= 0)
+        for (int i = 0; i < 4; i++) ol[i] = pa.out_layout[i];
+    if (!(ol[0] == 0 && ol[1] == 2 && ol[2] == 1 && ol[3] == 3) || ov.buf < 0 || ov.count() != rows * DIM) return -1;
+    if (buffer_reads(g, qkv, ai) != 0) return -1;
+    const auto xr = value_range(P, x), o = value_range(P, att);
+    return xr.first < o.second && o.first < xr.second ? -1 : ai;  // (views of the output share its buffer)
+}
+
+void plan_fused_attention(sox_graph& g) {
+    for (auto& kv : g.ln_fold) {
+        const int qi = kv.first, ai = fusable_attention(g, qi, g.plan.nodes[qi].in[0]);
+        if (ai < 0) continue;
         g.qkv_attn[qi] = ai;
         g.folded.insert(ai);
     }

@@ -1,17 +1,15 @@
-// Implicit-GEMM Conv2d / ConvTranspose instances of the LDS-DMA persistent ring (gemm_ring.h).
+// Implicit-GEMM Conv2d / ConvTranspose instances of the LDS-DMA persistent ring (gemm_ring.h): fp16 NHWC,
+// ic % 8 == 0, constant-0 or reflect padding.
 #include "gemm_ring.h"
 
-// implicit-GEMM Conv2d on the same ring (fp16 NHWC, ic % 8 == 0, constant-0 or reflect padding)
-SOX_CONV(sox_conv_f16_128x32_k32s4, half_t, 128, 32, 32, 32, 32, 4, 4, 2, 4)
+// few tiles: four stages of 64 or 32 input channels (32 where a 64-channel block would be half zeros)
 SOX_CONV(sox_conv_f16_64x64_k32s4, half_t, 64, 64, 32, 32, 32, 4, 4, 2, 4)
-SOX_CONV(sox_conv_f16_128x64_k32s4, half_t, 128, 64, 32, 64, 32, 4, 4, 2, 4)
-SOX_CONV(sox_conv_f16_128x128_k32s4, half_t, 128, 128, 32, 64, 64, 4, 4, 2, 4)
 SOX_CONV(sox_conv_f16_64x64_k64s4, half_t, 64, 64, 64, 32, 32, 4, 4, 2, 4)
-SOX_CONV(sox_conv_f16_128x64_k64s3, half_t, 128, 64, 64, 64, 32, 3, 4, 1, 4)
-// deep K (3x3 convs over many channels): more slices in flight per workgroup
-SOX_CONV(sox_conv_f16_128x32_k64s6, half_t, 128, 32, 64, 32, 32, 6, 4, 1, 4)
-SOX_CONV(sox_conv_f16_64x64_k64s8, half_t, 64, 64, 64, 32, 32, 8, 4, 1, 4)
-SOX_CONV(sox_conv_f16_128x64_k64s5, half_t, 128, 64, 64, 64, 32, 5, 4, 1, 4)
+// many tiles: two stages, two or three workgroups per CU; 96-wide tiles for 72..96, 168..192 .. channels
+SOX_CONV(sox_conv_f16_128x64_k64s2, half_t, 128, 64, 64, 64, 32, 2, 4, 3, 4)
+SOX_CONV(sox_conv_f16_128x96_k32s2, half_t, 128, 96, 32, 32, 96, 2, 4, 3, 4)
+SOX_CONV(sox_conv_f16_128x96_k64s2, half_t, 128, 96, 64, 32, 96, 2, 4, 2, 4)
+SOX_CONV(sox_conv_f16_128x128_k64s2, half_t, 128, 128, 64, 64, 64, 2, 4, 2, 4)
 // large convs (many output pixels, K >= 1024): the headline Gemm's 8-wave tilings, LDS-staged epilogue
 SOX_CONV_E(sox_conv_f16_256x128_w8k64s2, half_t, 256, 128, 64, 64, 64, 2, 8, 1, 4)
 // 256 output channels: the whole N in one tile (fewer DMA and LDS bytes per MFMA than 256 x 128); its

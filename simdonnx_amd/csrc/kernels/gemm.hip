@@ -1,4 +1,5 @@
-// Dense fp16 Gemm instances of the LDS-DMA persistent ring (gemm_ring.h).
+// Dense fp16 Gemm instances of the LDS-DMA persistent ring (gemm_ring.h): the 256-row tiles (the smaller
+// ones are gemm_small.hip's).
 #include "gemm_ring.h"
 
 // name: BMxBN tile, kBK slice depth, sSTAGES, wNW waves (4 when absent); SOX_GEMM_E: epilogue through LDS
@@ -11,18 +12,6 @@ SOX_GEMM(sox_gemm_f16_256x256_w8k64s2, half_t, 256, 256, 64, 128, 64, 2, 8, 1, 4
 SOX_GEMM(sox_gemm_f16_256x128_k32s3, half_t, 256, 128, 32, 128, 64, 3, 4, 2, 4)
 SOX_GEMM(sox_gemm_f16_256x128_k32s5, half_t, 256, 128, 32, 128, 64, 5, 4, 1, 4)
 SOX_GEMM_E(sox_gemm_f16_256x128_w8k64s2, half_t, 256, 128, 64, 64, 64, 2, 8, 1, 4)
-SOX_GEMM(sox_gemm_f16_128x128_k64s2, half_t, 128, 128, 64, 64, 64, 2, 4, 2, 4)
-SOX_GEMM(sox_gemm_f16_128x128_k32s4, half_t, 128, 128, 32, 64, 64, 4, 4, 2, 4)
-SOX_GEMM(sox_gemm_f16_128x64_k64s2, half_t, 128, 64, 64, 64, 32, 2, 4, 3, 4)
-SOX_GEMM(sox_gemm_f16_64x64_k64s2, half_t, 64, 64, 64, 32, 32, 2, 4, 4, 4)
-// short K (a few slices): every slice of a tile in flight from the start
-SOX_GEMM_E(sox_gemm_f16_64x64_k64s4, half_t, 64, 64, 64, 32, 32, 4, 4, 2, 4)
-SOX_GEMM(sox_gemm_f16_128x64_k64s4, half_t, 128, 64, 64, 64, 32, 4, 4, 1, 4)
-// A rows through a LayerNorm folded into the Gemm (the default tilings)
-SOX_GEMM_LN(sox_gemm_ln_f16_256x128_w8k64s2, half_t, 256, 128, 64, 64, 64, 2, 8, 1, 4, true)
-SOX_GEMM_LN(sox_gemm_ln_f16_128x128_k64s2, half_t, 128, 128, 64, 64, 64, 2, 4, 2, 4, false)
-SOX_GEMM_LN(sox_gemm_ln_f16_128x64_k64s2, half_t, 128, 64, 64, 64, 32, 2, 4, 3, 4, false)
-SOX_GEMM_LN(sox_gemm_ln_f16_64x64_k64s4, half_t, 64, 64, 64, 32, 32, 4, 4, 2, 4, true)
 
 // Matrix-core rate probe (bench.py --only mfma_peak): every wave runs `iters` rounds of four
 // independent v_mfma_f32_32x32x16_f16 chains on register operands, with operand bits from a per-lane

@@ -53,6 +53,24 @@ template <int I, int N, class F> SOX_DEV void static_for(F&& f) {
 template <int CPR> SOX_DEV int swz(int r) { return (r / (16 / CPR)) % CPR; }
 
 
+// The activation of an output stored as T (ACT < 0: the runtime `act`): gelu_fast belongs to 16-bit outputs.
+template <typename T, int ACT> SOX_DEV float out_act(float v, int act) {
+    if constexpr (sizeof(T) == 4) return sox_act(v, ACT >= 0 ? ACT : act);
+    if constexpr (ACT == SOX_ACT_GELU) return gelu_fast(v);
+    if constexpr (ACT >= 0) return sox_act(v, ACT);
+    return act_fast(v, act);
+}
+
+// One k-step of a 32x32 block from 16 bytes of each operand per lane: 16 k of a 16-bit type, or 8 k of fp32
+// as four 32x32x2 products (lanes 0-31 hold k 0..3, lanes 32-63 k 4..7; product e takes k e and 4 + e).
+SOX_DEV float16v mfma_step(half8 a, half8 b, float16v c) { return mfma32x32x16(a, b, c); }
+SOX_DEV float16v mfma_step(bf16x8 a, bf16x8 b, float16v c) { return mfma32x32x16(a, b, c); }
+SOX_DEV float16v mfma_step(float4v a, float4v b, float16v c) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+}
+
 // Epilogue of one wave's WM x WN block: lane l (l32 = l % 32, hl = l / 32) of 32x32 block (j, i) holds
 // output row m0 + 32 i + l32 and, for q = 0..3, channels n0 + 32 j + 8 q + 4 hl .. +3 in accumulator
 // elements 4q .. 4q+3 (the bias is already in the accumulators): activation on a float4, one 8-byte
@@ -82,7 +100,7 @@ SOX_DEV void store_tile(T* __restrict__ Y, const T* __restrict__ R, int ldy, int
     const bool aligned = pad_rows ? (ldy & 3) == 0 : ((ldy | N) & 3) == 0;
     if (convt) {  // uniform: ConvTranspose output, no residual
         const ConvtOut* ct = &ctv;
-        auto fin = [&](float a) { return ACT == SOX_ACT_GELU ? gelu_fast(a) : ACT >= 0 ? sox_act(a, ACT) : act_fast(a, act); };
+        auto fin = [&](float a) { return out_act<T, ACT>(a, act); };
         static_for<0, TJ * TI>([&](auto ji) {
             constexpr int j = decltype(ji)::value / TI, i = decltype(ji)::value % TI;
             const int m = m0 + i * 32 + l32;
@@ -122,10 +140,11 @@ SOX_DEV void store_tile(T* __restrict__ Y, const T* __restrict__ R, int ldy, int
     // lanes l and l + 32 hold channels 8q .. 8q+3 and 8q+4 .. 8q+7 of one row, so after converting q
     // pairs (2p, 2p+1) to 16-bit, one v_permlane32_swap per dword gives lane l all 8 channels of group
     // 2p and lane l + 32 all 8 of group 2p+1: one 16-byte store each instead of two 8-byte ones
-    if (WIDE && !R && (ldy & 7) == 0 && n0 + TJ * 32 <= N) {
+    if constexpr (WIDE && sizeof(T) == 2)
+    if (!R && (ldy & 7) == 0 && n0 + TJ * 32 <= N) {
         typedef vec_t<unsigned, 2> U2;
         typedef vec_t<unsigned, 4> U4;
-        auto fin = [&](float a) { return ACT == SOX_ACT_GELU ? gelu_fast(a) : ACT >= 0 ? sox_act(a, ACT) : act_fast(a, act); };
+        auto fin = [&](float a) { return out_act<T, ACT>(a, act); };
         static_for<0, TJ * TI>([&](auto ji) {
             constexpr int j = decltype(ji)::value / TI, i = decltype(ji)::value % TI;
             const int m = m0 + i * 32 + l32;
@@ -188,7 +207,7 @@ SOX_DEV void store_tile(T* __restrict__ Y, const T* __restrict__ R, int ldy, int
                 constexpr int e = decltype(ee)::value;
                 float v = acc[j][i][4 * q + e];
                 if (R) v += (float)rv[q][e];
-                h[e] = (T)fp32_value(ACT == SOX_ACT_GELU ? gelu_fast(v) : ACT >= 0 ? sox_act(v, ACT) : act_fast(v, act));
+                h[e] = (T)fp32_value(out_act<T, ACT>(v, act));
             });
             if (m < M && n < N) {
                 T* yp = Y + (long)m * ldy + n;
@@ -218,7 +237,7 @@ SOX_DEV void store_tile_lds(T* __restrict__ Y, int ldy, int M, int N, int m0, in
     typedef vec_t<T, 4> T4;
     typedef vec_t<T, 8> T8;
     const int lane = threadIdx.x & 63, l32 = lane & 31, hl = lane >> 5;
-    auto fin = [&](float a) { return ACT == SOX_ACT_GELU ? gelu_fast(a) : ACT >= 0 ? sox_act(a, ACT) : act_fast(a, act); };
+    auto fin = [&](float a) { return out_act<T, ACT>(a, act); };
     static_for<0, TI * ((TJ + 1) / 2)>([&](auto ip) {
         constexpr int i = decltype(ip)::value / ((TJ + 1) / 2), j0 = 2 * (decltype(ip)::value % ((TJ + 1) / 2));
         constexpr int JG = j0 + 1 < TJ ? 2 : 1, CH = JG * 4;  // blocks staged together, 16-byte chunks per row
@@ -264,14 +283,16 @@ constexpr int dma_chunk(int share) {
 // math) and a lane's source is its row's offset + the tap's offset + its channel. Channels past ic (the last block of a tap
 // when BK does not divide ic) and zero-padding taps are fetched from p.zeros; ic % 8 == 0. Rows past
 // M re-read row M - 1 (never stored).
+// KT (dense): K is any multiple of 8; the last slice's chunks past K are fetched from p.zeros.
 template <typename T, int BM, int BN, int BK, int WM, int WN, int STAGES, int NW, int GM, bool CONV = false,
-          bool EPI_LDS = false, bool LN = false, int CPARTS = 0, bool LARGE = false>
+          bool EPI_LDS = false, bool LN = false, int CPARTS = 0, bool LARGE = false, bool KT = false>
 __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
-    typedef vec_t<T, 8> T8;
+    constexpr int CE = 16 / sizeof(T);          // elements of a 16-byte chunk
+    typedef vec_t<T, CE> T8;                    // a chunk: one operand of a k-step per lane
     typedef vec_t<T, 2> T2;
-    constexpr int CPR = BK / 8;                 // 16-byte chunks per LDS row
-    constexpr int ROWB = BK * 2;                // LDS row bytes
-    constexpr int KS = BK / 16;                 // MFMA k-steps per slice
+    constexpr int CPR = BK / CE;                // 16-byte chunks per LDS row
+    constexpr int ROWB = BK * sizeof(T);        // LDS row bytes
+    constexpr int KS = CPR / 2;                 // MFMA k-steps per slice
     constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, BIAS_BYTES = BN * 4;
     constexpr int STAGE_BYTES = A_BYTES + B_BYTES + BIAS_BYTES;
     constexpr int BIAS_LANES = BIAS_BYTES / 16 / NW;  // lanes of each wave's bias DMA (16 B each)
@@ -285,7 +306,8 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
     constexpr bool BIAS_ONCE = STAGES == 2;
     constexpr int TI = WM / 32, TJ = WN / 32;   // 32x32 MFMA blocks: m (columns) x n (rows)
     constexpr int WAVES_N = BN / WN;
-    static_assert(CPR == 4 || CPR == 8, "BK = 32 or 64");
+    static_assert(CPR == 4 || CPR == 8, "64 or 128 bytes of K per slice");
+    static_assert(sizeof(T) == 2 || (!EPI_LDS && !LN), "fp32: plain register epilogue");
     static_assert(KS % 2 == 0, "fragment sets alternate per k-step and must realign per slice");
     static_assert((BM / WM) * (BN / WN) == NW && WM % 32 == 0 && WN % 32 == 0, "tiling");
     static_assert(A_IT * CH_A * NW == A_BYTES && B_IT * CH_B * NW == B_BYTES && CH_A % 16 == 0 && CH_B % 16 == 0,
@@ -315,7 +337,8 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
     // with LN the bias is added after the normalisation, so the accumulators start from zero
     const bool has_bias = (p.flags & SOX_F_BIAS) != 0 && !(CONV && (p.flags & SOX_F_CONVT)) && !LN;
     const int cblocks = CONV ? (p.ic + BK - 1) / BK : 1;  // channel blocks per tap
-    const int nk = CONV ? p.kh * p.kw * cblocks : K / BK;
+    static_assert(!KT || (!CONV && !LN), "K tail: plain dense Gemm only");
+    const int nk = CONV ? p.kh * p.kw * cblocks : KT ? (K + BK - 1) / BK : K / BK;
     const long img_elems = CONV ? (long)p.ih * p.iw * p.ic : 0;  // conv: elements of one input image
     const bool reflect = (p.flags & SOX_F_REFLECT) != 0;
 
@@ -375,21 +398,24 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
                 else
                     a_img[i] = A + (long)b * img_elems;
             } else {
-                a_src[i] = A + (long)min(bm + r, M - 1) * p.lda + a_chunk(i) * 8;
+                a_src[i] = A + (long)min(bm + r, M - 1) * p.lda + a_chunk(i) * CE;
             }
         }
 #pragma unroll
         for (int i = 0; i < B_IT; i++) {
             const int r = ((wave * B_IT + i) * CH_B + lane * 16) / ROWB;
             if constexpr (CONV)
-                b_o[i] = min(bn + r, N - 1) * p.kpad + b_chunk(i) * 8;  // W < 2^31 elements (the launcher checks)
+                b_o[i] = min(bn + r, N - 1) * p.kpad + b_chunk(i) * CE;  // W < 2^31 elements (the launcher checks)
             else
-                b_src[i] = W + (long)min(bn + r, N - 1) * p.kpad + b_chunk(i) * 8;
+                b_src[i] = W + (long)min(bn + r, N - 1) * p.kpad + b_chunk(i) * CE;
         }
     };
-    // ring slice gs = (index in this workgroup's tile list) * nk + k-slice. Slices past the end are
-    // still issued (re-reading the last tile's rows into a stage nobody reads again), so every slice
-    // has the same number of loads in flight and one static vmcnt covers them all.
+    // ring slice gs = (index in this workgroup's tile list) * nk + k-slice. The 8-wave instances issue
+    // slices past the end too (re-reading the last tile's rows into a stage nobody reads again), so that
+    // every slice has the same number of loads in flight, one static vmcnt covers them all and the k-steps
+    // stay one basic block. The 4-wave instances (TRIM) serve short reductions, where STAGES junk slices
+    // cost as much as the real ones: they issue none, and their last waits count the slices left.
+    // Detector at 960 698 -> 686 us, MobileNetV3 at 640 391 -> 379 us.
     // prep computes a slice's DMA sources (calling set_sources at a tile's first slice), fire issues
     // the DMAs.
     struct Src {
@@ -405,19 +431,34 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
     struct Tap {
         int tap, c0, ky, kx, off;
     };
-    auto slice_tap = [&](int gs) __attribute__((always_inline)) {
-        Tap t;
-        const int kt = gs % nk, taps = p.kh * p.kw, cb = kt / taps;
-        t.tap = kt - cb * taps;
-        t.c0 = cb * BK;
-        t.ky = t.tap / p.kw;
-        t.kx = t.tap - t.ky * p.kw;
-        t.off = (t.ky * p.iw + t.kx) * p.ic;
-        return t;
+    // The slice being issued, as running scalar counters: its k-slice and tile and (conv) its tap and first
+    // channel. Slices are issued in order, so each starts from the one before it; divisions of the slice
+    // number by nk, kh * kw and kw cost a conv slice ~0.1 us (5x5 48 -> 56 over 8x50x70, 50 slices: 29.4 ->
+    // 22.4 us; 3x3 256 -> 256 over 30x40, 36 slices: 22.9 -> 19.8 us).
+    int i_kt = nk - 1, i_tile = vid - G, i_ky = p.kh - 1, i_kx = p.kw - 1, i_c0 = 0;
+    auto slice_tap = [&]() __attribute__((always_inline)) {
+        return Tap{i_ky * p.kw + i_kx, i_c0, i_ky, i_kx, (i_ky * p.iw + i_kx) * p.ic};
+    };
+    // starts slice gs (the one after the last started): a tile's first slice sets its sources
+    auto start_slice = [&](int gs) __attribute__((always_inline)) {
+        if (++i_kt == nk) {
+            i_kt = 0;
+            i_tile += G;
+            if (gs < total) set_sources(i_tile);
+            i_ky = i_kx = i_c0 = 0;
+        } else if constexpr (CONV) {
+            if (++i_kx == p.kw) {
+                i_kx = 0;
+                if (++i_ky == p.kh) {
+                    i_ky = 0;
+                    i_c0 += BK;
+                }
+            }
+        }
     };
     // conv DMA source of A instruction i / B instruction i for a slice
     auto conv_a = [&](int i, const Tap& t) __attribute__((always_inline)) {
-        const int ch = t.c0 + a_chunk(i) * 8;
+        const int ch = t.c0 + a_chunk(i) * CE;
         const int iy = (int)(a_yx[i] >> 16) - 32768 + t.ky, ix = (int)(a_yx[i] & 0xffffu) - 32768 + t.kx;
         bool ok = (unsigned)iy < (unsigned)p.ih && (unsigned)ix < (unsigned)p.iw;
         int off = a_off0[i] + t.off + ch;
@@ -434,24 +475,32 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
         return ok ? a_img[i] + off : Z;  // one image < 2^31 elements
     };
     auto conv_b = [&](int i, const Tap& t) __attribute__((always_inline)) {
-        const int ch = t.c0 + b_chunk(i) * 8;
+        const int ch = t.c0 + b_chunk(i) * CE;
         return ch < p.ic ? W + b_o[i] + t.tap * p.ic + t.c0 : Z;  // b_o includes the chunk
     };
+    // dense sources of a slice from k0: past K (KT, the last slice) the zero block
+    auto dense_a = [&](int i, int k0) __attribute__((always_inline)) {
+        if constexpr (KT) return k0 + a_chunk(i) * CE < K ? a_src[i] + k0 : Z;
+        return a_src[i] + k0;
+    };
+    auto dense_b = [&](int i, int k0) __attribute__((always_inline)) {
+        if constexpr (KT) return k0 + b_chunk(i) * CE < K ? b_src[i] + k0 : Z;
+        return b_src[i] + k0;
+    };
     auto prep = [&](int gs, Src& q) __attribute__((always_inline)) {
-        const int kt = gs % nk;
-        if (kt == 0 && gs < total) set_sources(vid + (gs / nk) * G);
+        start_slice(gs);
         if constexpr (CONV) {
-            const Tap t = slice_tap(gs);
+            const Tap t = slice_tap();
 #pragma unroll
             for (int i = 0; i < A_IT; i++) q.a[i] = conv_a(i, t);
 #pragma unroll
             for (int i = 0; i < B_IT; i++) q.b[i] = conv_b(i, t);
         } else {
-            const int k0 = kt * BK;
+            const int k0 = i_kt * BK;
 #pragma unroll
-            for (int i = 0; i < A_IT; i++) q.a[i] = a_src[i] + k0;
+            for (int i = 0; i < A_IT; i++) q.a[i] = dense_a(i, k0);
 #pragma unroll
-            for (int i = 0; i < B_IT; i++) q.b[i] = b_src[i] + k0;
+            for (int i = 0; i < B_IT; i++) q.b[i] = dense_b(i, k0);
         }
         q.c = c_src;
     };
@@ -466,7 +515,7 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
                 __builtin_amdgcn_global_load_lds(q.b[i], LDS_PTR(st + A_BYTES + (wave * B_IT + i) * CH_B), 16, 0, 0);
         // the tile's bias rides along with its first slice (with every slice when the in-loop waits
         // count loads: more than two stages); the accumulators of a new tile start from it
-        if (lane < BIAS_LANES && (!BIAS_ONCE || gs % nk == 0))
+        if (lane < BIAS_LANES && (!BIAS_ONCE || i_kt == 0))
             __builtin_amdgcn_global_load_lds(q.c, LDS_PTR(st + A_BYTES + B_BYTES + wave * BIAS_LANES * 16), 16, 0, 0);
     };
     auto issue = [&](int gs) __attribute__((always_inline)) {
@@ -481,29 +530,28 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
     // slice's vmcnt wait (one part per k-step over all four k-steps left the last part too little time).
     // Every part of slice g + STAGES - 1 is out before the vmcnt wait of slice g, so the waits count the
     // same loads as before.
-    constexpr bool SPREAD = (!CONV || CPARTS > 1) && KS >= 2;
+    constexpr bool TRIM = NW == 4;
+    constexpr bool SPREAD = (!CONV || CPARTS > 1) && KS >= 2 && !TRIM;
     constexpr int NPARTS = !SPREAD ? 1 : CONV ? (CPARTS < KS ? CPARTS : KS) : 2;
     constexpr int PER = (LOADS + NPARTS - 1) / NPARTS;  // DMA instructions per part
     auto fire_part = [&](int gs, auto pp) __attribute__((always_inline)) {
         constexpr int p0 = decltype(pp)::value * PER;
-        if constexpr (p0 == 0) {
-            if (gs % nk == 0 && gs < total) set_sources(vid + (gs / nk) * G);
-        }
-        const int k0 = (gs % nk) * BK;
+        if constexpr (p0 == 0) start_slice(gs);
+        const int k0 = i_kt * BK;
         Tap t{};
-        if constexpr (CONV) t = slice_tap(gs);  // recomputed per part: scalar work, no registers held
+        if constexpr (CONV) t = slice_tap();
         unsigned char* st = smem + (gs % STAGES) * STAGE_BYTES;
         static_for<p0, (p0 + PER < LOADS ? p0 + PER : LOADS)>([&](auto xx) {
             constexpr int x = decltype(xx)::value;
             if constexpr (x < A_IT) {
-                const T* src = CONV ? conv_a(x, t) : a_src[x] + k0;
+                const T* src = CONV ? conv_a(x, t) : dense_a(x, k0);
                 if (a_lane) __builtin_amdgcn_global_load_lds(src, LDS_PTR(st + (wave * A_IT + x) * CH_A), 16, 0, 0);
             } else if constexpr (x < A_IT + B_IT) {
-                const T* src = CONV ? conv_b(x - A_IT, t) : b_src[x - A_IT] + k0;
+                const T* src = CONV ? conv_b(x - A_IT, t) : dense_b(x - A_IT, k0);
                 if (b_lane)
                     __builtin_amdgcn_global_load_lds(src, LDS_PTR(st + A_BYTES + (wave * B_IT + x - A_IT) * CH_B), 16, 0, 0);
             } else {
-                if (lane < BIAS_LANES && (!BIAS_ONCE || gs % nk == 0))
+                if (lane < BIAS_LANES && (!BIAS_ONCE || i_kt == 0))
                     __builtin_amdgcn_global_load_lds(c_src, LDS_PTR(st + A_BYTES + B_BYTES + wave * BIAS_LANES * 16), 16, 0, 0);
             }
         });
@@ -524,9 +572,18 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
         b_off[j] = A_BYTES + r * ROWB + ((hl ^ swz<CPR>(r)) << 4);
     }
 
+    // waits until all but the newest min(MAX, left) slices' loads have landed
+    auto wait_slices = [&](auto max_slices, int left) __attribute__((always_inline)) {
+        constexpr int MAX = decltype(max_slices)::value;
+        static_for<0, MAX + 1>([&](auto rr) {
+            constexpr int r = decltype(rr)::value;
+            if (r == MAX ? left >= r : r == 0 ? left <= 0 : left == r) wait_vmcnt<r * LOADS>();
+        });
+    };
     if (total == 0) return;
     int bm_cur, bn_cur;  // origin of the tile being multiplied
     tile_origin(vid, bm_cur, bn_cur);
+    int m_kt = 0, m_tile = vid;  // its k-slice and number
 
     float16v acc[TJ][TI];
     T8 fa0[TI], fb0[TJ], fa1[TI], fb1[TJ];
@@ -605,7 +662,7 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
                 default: store_tile_lds<T, -1>(Y, p.ldy, M, N, bm_cur + wm0, bn_cur + wn0, acc, act, stg); break;
                 }
                 if (gs + 1 < total) {
-                    tile_origin(vid + (gs + 1) / nk * G, bm_cur, bn_cur);
+                    tile_origin(m_tile += G, bm_cur, bn_cur);
                     init_acc(gs + 1);
                 }
                 return;
@@ -618,15 +675,23 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
         default: store_tile<T, -1, TJ, TI, CONV, LARGE>(Y, R, p.ldy, M, N, bm_cur + wm0, bn_cur + wn0, acc, act, ctp, cto, pad_rows, ru); break;
         }
         if (gs + 1 < total) {
-            tile_origin(vid + (gs + 1) / nk * G, bm_cur, bn_cur);
+            tile_origin(m_tile += G, bm_cur, bn_cur);
             init_acc(gs + 1);  // published by this slice's barrier
         }
     };
 
 #pragma unroll
-    for (int s = 0; s < STAGES; s++) issue(s);
+    for (int s = 0; s < STAGES; s++)
+        if (!TRIM || s < total) issue(s);
     // slice 0 (loads complete in order; slice 1 carries LOADS - 1 of them when it does not start a tile)
-    wait_vmcnt<(STAGES - 1) * LOADS - (BIAS_ONCE ? 1 : 0)>();
+    if (TRIM && total < STAGES) {
+        if constexpr (STAGES > 2)
+            wait_slices(std::integral_constant<int, STAGES - 2>{}, total - 1);
+        else
+            wait_vmcnt<0>();
+    } else {
+        wait_vmcnt<(STAGES - 1) * LOADS - (BIAS_ONCE ? 1 : 0)>();
+    }
     __builtin_amdgcn_s_barrier();
     init_acc(0);
     read_step(0, 0, fa0, fb0);
@@ -640,21 +705,27 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
             if constexpr (s == KS - 1) {
                 // slice gs+1 landed (this wave's loads; later slices may stay in flight) and every read
                 // of slice gs done; after the barrier both hold for all waves
-                wait_vmcnt<(STAGES - 2) * LOADS>();
-                wait_lgkmcnt0();
-                __builtin_amdgcn_s_barrier();
-                // into stage gs % STAGES; may already be a later tile's slice
-                if constexpr (SPREAD)
-                    fire_part(gs + STAGES, std::integral_constant<int, 0>{});
-                else
-                    issue(gs + STAGES);
+                // the refill goes into stage gs % STAGES; may already be a later tile's slice
+                if (!TRIM || gs + STAGES < total) {
+                    wait_vmcnt<(STAGES - 2) * LOADS>();
+                    wait_lgkmcnt0();
+                    __builtin_amdgcn_s_barrier();
+                    if constexpr (SPREAD)
+                        fire_part(gs + STAGES, std::integral_constant<int, 0>{});
+                    else
+                        issue(gs + STAGES);
+                } else {
+                    wait_slices(std::integral_constant<int, STAGES - 2>{}, total - 2 - gs);
+                    wait_lgkmcnt0();
+                    __builtin_amdgcn_s_barrier();
+                }
                 read_step(gs + 1, 0, na, nb);
             } else {
                 read_step(gs, s + 1, na, nb);
             }
             static_for<0, TJ * TI>([&](auto ji) {
                 constexpr int j = decltype(ji)::value / TI, i = decltype(ji)::value % TI;
-                acc[j][i] = mfma32x32x16(cb[j], ca[i], acc[j][i]);
+                acc[j][i] = mfma_step(cb[j], ca[i], acc[j][i]);
             });
             if constexpr (SPREAD && s + 1 < NPARTS && (s + 1) * PER < LOADS) {
                 // part s + 1 of the slice whose part 0 went out after the last barrier (the prologue
@@ -677,7 +748,7 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
             }
             // MFMA, read, MFMA, read, ...: this step's operands were read one step earlier, and the
             // next step's reads issue while the matrix pipe works through this step
-            constexpr int RD = TI + TJ, MF = TI * TJ;
+            constexpr int RD = TI + TJ, MF = TI * TJ * (sizeof(T) == 4 ? 4 : 1);
             if constexpr (!CONV) {
                 // dense Gemm: the DMA instructions this step issues (a part after the barrier or after a
                 // k-step) go one after each MFMA, so a wave that stalls on DMA issue has MFMAs of its own
@@ -707,9 +778,12 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
             __builtin_amdgcn_sched_barrier(0);
         });
         wait_lgkmcnt0();  // next slice's first fragments (read before this slice's last MFMAs)
-        if (gs % nk == nk - 1) epilogue(gs);
+        if (++m_kt == nk) {
+            m_kt = 0;
+            epilogue(gs);
+        }
     }
-    wait_vmcnt<0>();  // the trailing (unused) slices land before the workgroup's LDS is released
+    if (!TRIM) wait_vmcnt<0>();  // the trailing (unused) slices land before the workgroup's LDS is released
 }
 
 // T: the 16-bit storage type (half_t or bf16_t)
@@ -721,6 +795,11 @@ __device__ __forceinline__ void gemm_body(const sox_igemm_args& p) {
 #define SOX_GEMM_E(NAME, T, BM, BN, BK, WM, WN, ST, NW, OCC, GM)                                    \
     extern "C" __global__ void __launch_bounds__(64 * NW, OCC) NAME(sox_igemm_args p) {           \
         gemm_body<T, BM, BN, BK, WM, WN, ST, NW, GM, false, true>(p);                             \
+    }
+// any K that is a multiple of 8 (the last slice's tail from the zero block); E = epilogue through LDS
+#define SOX_GEMM_KT(NAME, T, BM, BN, BK, WM, WN, ST, NW, OCC, GM, E)                                \
+    extern "C" __global__ void __launch_bounds__(64 * NW, OCC) NAME(sox_igemm_args p) {           \
+        gemm_body<T, BM, BN, BK, WM, WN, ST, NW, GM, false, E, false, 0, false, true>(p);         \
     }
 // A rows LayerNorm'ed on the fly (the LayerNorm folded into the Gemm); E = epilogue through LDS
 #define SOX_GEMM_LN(NAME, T, BM, BN, BK, WM, WN, ST, NW, OCC, GM, E)                               \

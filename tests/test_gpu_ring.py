@@ -1,0 +1,112 @@
+"""The LDS-DMA ring at the sizes where its tilings, tails and trimmed rings can go wrong, against the
+oracle: K tails (a multiple of 8 that is not one of 64), N that no group of 4 divides, single
+rows, reductions of one slice up to more than the ring's stages, every tiling the estimate can pick
+(through shapes that pick it), 1x1 convs as dense products.
+
+Tolerances: 16-bit outputs are one rounding of an fp32 sum (2^-11 / 2^-8 relative to the element, whose
+magnitude is at most the maximum); the fp32 sums of K terms differ in order only, at most K 2^-24 of the sum
+of magnitudes, which for these operands is within 30 times the largest result."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import max_rel
+from oracle.interp import _bf16
+from simdonnx_amd import synth
+from simdonnx_amd.backend import HipInferenceSession
+from simdonnx_amd.plan import NHWC, PlanBuilder
+
+pytestmark = pytest.mark.gpu
+
+
+def stored(a, storage):
+    a = np.asarray(a, np.float32)
+    return a if storage == "f32" else _bf16(a) if storage == "bf16" else a.astype(np.float16).astype(np.float32)
+
+
+def tol(storage, k):
+    return {"f32": 30 * k * 2.0**-24, "f16": 1e-3, "bf16": 8e-3}[storage]
+
+
+def run(hip, plan, ins, storage):
+    g = hip.graph(plan, storage)
+    kernels = g.kernels
+    with HipInferenceSession(g) as s:
+        for i, x in enumerate(ins):
+            s.set_input(x, i)
+        return s.run().copy(), kernels
+
+
+GEMMS = [(1, 8, 1), (1, 64, 64), (3, 16, 5), (64, 24, 64), (47, 40, 88), (65, 72, 97), (33, 120, 6), (130, 200, 200),
+         (256, 1000, 96), (200, 520, 190), (40, 192, 768), (63, 768, 192), (786, 760, 760), (900, 16, 300), (2000, 24, 96),
+         (6000, 320, 640), (6016, 328, 1288), (3000, 136, 1000), (4096, 264, 768), (12300, 40, 192), (16640, 200, 384)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("case", GEMMS, ids=lambda c: "x".join(map(str, c)))
+def test_gemm_tails_and_tilings(hip, storage, case):
+    m, k, n = case
+    x = stored(synth.normal(141, 1, (m, k), 1.0), storage)
+    w = stored(synth.normal(141, 2, (k, n), k**-0.5), storage)
+    b = synth.uniform(141, 3, (n,), -0.5, 0.5)
+    r = stored(synth.normal(141, 4, (m, n), 1.0), storage)
+    for act, bias, residual in (("gelu", True, False), ("none", False, True)):
+        pb = PlanBuilder()
+        xv, rv = pb.input((m, k), None, "x"), pb.input((m, n), None, "r")
+        y = pb.gemm(xv, w, b if bias else None, act=act, name="gemm")
+        y = pb.add(rv, y, name="res") if residual else y
+        got, kernels = run(hip, pb.build(y), [x, r], storage)
+        print(f"[gpu] {storage} {case} {kernels[0]}", flush=True)
+        assert len(kernels) == 1 and "igemm" not in kernels[0], kernels
+        want = O.gemm(x, w, b if bias else None, act=act)
+        assert max_rel(got, want + r if residual else want) < tol(storage, k), kernels
+
+
+def test_every_default_tiling_is_reached(hip):
+    """The shapes above (and the wide products) cover every tiling that the estimate chooses from."""
+    kernels = set()
+    for storage in ("f16",):
+        for m, k, n in GEMMS + [(8192, 768, 3072), (4096, 1024, 2000), (4096, 1024, 1000), (8192, 760, 3000),
+                                (1024, 1536, 1024), (8192, 512, 512), (512, 384, 8192), (8192, 1016, 8192), (8192, 512, 1024)]:
+            pb = PlanBuilder()
+            y = pb.gemm(pb.input((m, k), None, "x"), np.zeros((k, n), np.float32), None, name="gemm")
+            g = hip.graph(pb.build(y), storage)
+            kernels.update(g.kernels)
+            g.release()
+    want = ["gemm_f16_256x192_w8k64s2", "gemm_f16_256x128_w8k64s2", "gemm_f16_128x64_k64s2e", "gemm_f16_64x64_k64s2",
+            "gemm_kt_f16_256x128_w8k64s2", "gemm_kt_f16_64x64_k64s2",
+            "gemm_kt_f16_128x96_k32s2", "gemm_kt_f16_64x64_k32s2"]
+    missing = [w for w in want if "sox_" + w not in kernels]
+    assert not missing, (missing, sorted(kernels))
+
+
+# (n, h, w, ic, oc, k, stride, act, residual, pad_mode)
+CONVS = [(1, 7, 9, 8, 8, 1, 1, "relu", False, 0), (2, 33, 31, 24, 88, 1, 1, "none", True, 0),
+         (1, 30, 41, 16, 72, 1, 1, "hardswish", False, 0), (2, 60, 60, 40, 240, 1, 1, "relu", False, 0),
+         (1, 20, 20, 576, 96, 1, 1, "none", True, 0), (1, 9, 11, 40, 80, 3, 1, "relu", False, 0),
+         (2, 47, 63, 96, 168, 3, 1, "hardswish", True, 0), (1, 15, 17, 72, 100, 3, 2, "none", False, 0),
+         (1, 40, 40, 64, 24, 5, 1, "relu", False, 0), (2, 40, 40, 128, 256, 3, 1, "gelu", False, 0),
+         (1, 31, 33, 96, 96, 3, 1, "relu", False, 1), (8, 50, 30, 48, 56, 5, 1, "none", False, 0),
+         (4, 64, 64, 40, 80, 3, 1, "relu", False, 0), (8, 64, 64, 128, 128, 3, 1, "relu", False, 0),
+         (1, 1, 5, 8, 9, 3, 1, "none", False, 0), (1, 12, 160, 64, 192, 1, 1, "none", False, 0)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("case", CONVS, ids=lambda c: "x".join(map(str, c)))
+def test_conv_tails_and_tilings(hip, storage, case, monkeypatch):
+    n, h, w, ic, oc, k, st, act, res, mode = case
+    monkeypatch.setenv("SIMDONNX_HIP_NOHALO", "1")  # every 3x3 through the ring
+    p = k // 2
+    oh, ow = (h + 2 * p - k) // st + 1, (w + 2 * p - k) // st + 1
+    x = stored(synth.normal(142, 1, (n, h, w, ic), 1.0), storage)
+    wt = stored(synth.normal(142, 2, (oc, ic, k, k), (k * k * ic)**-0.5), storage)
+    b = synth.uniform(142, 3, (oc,), -0.5, 0.5)
+    r = stored(synth.normal(142, 4, (n, oh, ow, oc), 1.0), storage) if res else None
+    pb = PlanBuilder()
+    ins = [pb.input((n, ic, h, w), NHWC, "x")] + ([pb.input((n, oc, oh, ow), NHWC, "r")] if res else [])
+    y = pb.conv(ins[0], wt, b, stride=st, pad=p, act=act, add=ins[1] if res else None, pad_mode=mode, name="conv")
+    got, kernels = run(hip, pb.build(y), [x] + ([r] if res else []), storage)
+    print(f"[gpu] {storage} {case} {kernels[0]}", flush=True)
+    assert len(kernels) == 1 and "igemm" not in kernels[0], kernels
+    want = O.conv(x, wt, b, r, stride=(st, st), pads=(p, p, p, p), act=act, pad_mode=mode)
+    assert max_rel(got, want) < tol(storage, k * k * ic), kernels
