@@ -715,6 +715,16 @@ struct Emitter {
             (uint32_t)(tm * tn), 1, 1, 256, 0, label);
     }
 
+    static constexpr const char* kF32Split = "sox_conv_f32_split";
+    // The fp32 32 x 32 tile with K split over its waves (conv_f32.hip)
+    void launch_f32_split(int node, const sox_igemm_args& a, sox_bind x, sox_bind w, sox_bind bias, sox_bind add_b,
+                          sox_bind y, const std::string& label) {
+        add(node, kF32Split, a,
+            {{offsetof(sox_igemm_args, x), x}, {offsetof(sox_igemm_args, w), w}, {offsetof(sox_igemm_args, bias), bias},
+             {offsetof(sox_igemm_args, add), add_b}, {offsetof(sox_igemm_args, y), y}, {offsetof(sox_igemm_args, zeros), none()}},
+            (uint32_t)((a.m + 31) / 32), (uint32_t)((a.n + 31) / 32), 1, 256, 0, label);
+    }
+
     // A tiling of the LDS-DMA ring and what it takes on MI355X, in us: with q tiles on the busiest CU and nk
     // slices of bk, base + q tile + nk max(lat, q thr). lat is a slice's DMA and barrier round trip when the
     // CU has one tile, thr a slice's share when several workgroups overlap theirs. The constants are fits to
@@ -760,7 +770,7 @@ struct Emitter {
     }
 
     // Dense product on the LDS-DMA ring (gemm_ring.h): a Gemm, or a 1x1 conv over its pixels. a holds m, n, k
-    // (a multiple of 8), ldy and the epilogue flags.
+    // (whole 16-byte chunks: a multiple of 8, fp32 of 4), ldy and the epilogue flags.
     void launch_gemm_dma(int node, sox_igemm_args a, sox_bind x, sox_bind w, sox_bind bias, sox_bind add_b, sox_bind y,
                          const sox_graph::LnFold* ln, const std::string& label) {
         static const RingCfg cfgs16[] = {
@@ -784,13 +794,28 @@ struct Emitter {
             {"sox_gemm_kt_f16_64x64_k64s2", 64, 64, 64, 4, 0.3f, 0.25f, 3.5f, 0.35f},
             {"sox_gemm_kt_f16_128x96_k32s2", 128, 96, 32, 3, 0.3f, 0.26f, 4.0f, 0.7f},
             {"sox_gemm_kt_f16_64x64_k32s2", 64, 64, 32, 4, 0.19f, 0.16f, 3.4f, 0.35f}};
+        static const RingCfg cfgs32[] = {
+            {"sox_gemm_f32_128x64_k32s2", 128, 64, 32, 3, 1.23f, 1.23f, 4.0f, 1.0f},
+            {"sox_gemm_f32_64x64_k32s2", 64, 64, 32, 4, 0.62f, 0.62f, 3.5f, 0.6f},
+            {"sox_gemm_f32_128x32_k32s2", 128, 32, 32, 4, 0.65f, 0.65f, 3.5f, 0.5f},
+            {kF32Split, 32, 32, 16, 2, 0.105f, 0.1f, 3.0f, 0.8f}};
         const char* forced = getenv("SIMDONNX_HIP_GEMM");
         const RingCfg* pick;
-        if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 6, 0, 6, a.m, a.n, a.k, 1, nullptr, "");
+        if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, nullptr, "");
+        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 6, 0, 6, a.m, a.n, a.k, 1, nullptr, "");
         else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5, a.m, a.n, a.k, 1, forced, "SIMDONNX_HIP_GEMM");
         a.kpad = pad8(a.k);
         a.lda = a.k;
         a.flags |= SOX_F_DENSE_A;
+        if (pick->name == kF32Split) {  // a 1x1 conv over the rows
+            a.ih = a.oh = 1;
+            a.iw = a.ow = a.m;
+            a.ic = a.k;
+            a.kh = a.kw = a.sh = a.sw = 1;
+            a.pt = a.pl = 0;
+            launch_f32_split(node, a, x, w, bias, add_b, y, label);
+            return;
+        }
         a.tiles_n = (a.n + pick->bn - 1) / pick->bn;
         std::string kname = pick->name;
         std::vector<std::pair<size_t, sox_bind>> ptrs = {
@@ -828,6 +853,11 @@ struct Emitter {
             // by the rules for large convs below
             {"sox_conv_f16_256x128_w8k64s2", 256, 128, 64, 1}, {"sox_conv_f16_256x256_w8k64s2", 256, 256, 64, 1},
             {"sox_conv_f16_h256", 256, 256, 64, 1}};
+        static const RingCfg cfgs32[] = {
+            {"sox_conv_f32_128x64_k32s2", 128, 64, 32, 3, 1.4f, 1.2f, 4.0f, 1.0f},
+            {"sox_conv_f32_64x64_k32s4", 64, 64, 32, 2, 0.73f, 0.7f, 3.5f, 0.6f},
+            {"sox_conv_f32_128x32_k32s2", 128, 32, 32, 4, 0.88f, 0.7f, 3.5f, 0.6f},
+            {kF32Split, 32, 32, 16, 2, 0.105f, 0.1f, 3.0f, 0.8f}};  // (zero padding only)
         // the ring keeps each row's receptive-field origin in 16 bits a coordinate and W offsets in 32
         if (a.ih > 30000 || a.iw > 30000) unsupported("conv: an image side over 30000 pixels");
         if ((int64_t)a.n * a.kpad >= (int64_t)1 << 31) unsupported("conv: weights of 2^31 elements or more");
@@ -846,20 +876,26 @@ struct Emitter {
         const char* name = nullptr;
         const char* forced = getenv("SIMDONNX_HIP_CONV");  // tuning / tests
         if (forced && *forced) name = forced;
-        else if (h256_ok && h256_tiles >= 2 * cus && !getenv("SIMDONNX_HIP_NO_H256"))
+        else if (g.f16 && h256_ok && h256_tiles >= 2 * cus && !getenv("SIMDONNX_HIP_NO_H256"))
             name = "sox_conv_f16_h256";
-        else if (a.ic % 64 == 0 && a.k >= 1024 && a.n % 256 == 0 && !(a.flags & SOX_F_CONVT) &&
+        else if (g.f16 && a.ic % 64 == 0 && a.k >= 1024 && a.n % 256 == 0 && !(a.flags & SOX_F_CONVT) &&
                  tiles(256, 256) >= 2 * cus && in32)
             // large convs over a multiple of 256 output channels: at least two rounds of 256x256 tiles
             // (8 waves of 128x64; 0.67x the DMA and 0.75x the LDS fragment bytes per MFMA of 256x128);
             // its DMA rows hold 32-bit offsets into the input
             name = "sox_conv_f16_256x256_w8k64s2";
-        else if (a.ic % 64 == 0 && a.k >= 1024 && a.n % 128 == 0 && !(a.flags & SOX_F_CONVT) &&
+        else if (g.f16 && a.ic % 64 == 0 && a.k >= 1024 && a.n % 128 == 0 && !(a.flags & SOX_F_CONVT) &&
                  tiles(256, 128) >= 2 * cus)
             // large convs: at least two rounds of 256x128 tiles on every CU, 8 waves each
             name = "sox_conv_f16_256x128_w8k64s2";
         const int64_t taps = (int64_t)a.kh * a.kw;
-        const RingCfg* c = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV");
+        const RingCfg* c =
+            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
+                  : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, nullptr, "");
+        if (c->name == kF32Split) {
+            launch_f32_split(node, a, x, w, bias, add_b, y, "conv");
+            return;
+        }
         if (!in32 && !strcmp(c->name, "sox_conv_f16_256x256_w8k64s2"))
             unsupported("conv: the 256x256 tile takes inputs of fewer than 2^31 elements");
         if (!strcmp(c->name, "sox_conv_f16_h256")) {
@@ -1046,6 +1082,13 @@ struct Emitter {
         a.lda = 0;
         char amode = ic % ld() == 0 ? 'v' : 's';
         const int st = p.strides[0];
+        // fp32 with a short reduction (conv_f32.hip)
+        const bool f32_short = !g.f16 && ic % 16 == 0 && a.k % 64 == 0 && a.k <= 576 && oc % 4 == 0 && a.ldy % 4 == 0 &&
+                               p.pad_mode == 0 && p.pad_value == 0.0f && !getenv("SIMDONNX_HIP_IGEMM");
+        // what the ring's packed origins and 32-bit offsets hold; larger fp32 convs stay on the implicit GEMM
+        const bool ring_f32_ok = ih <= 30000 && iw <= 30000 && (int64_t)ih * iw * ic < ((int64_t)1 << 31) &&
+                                 (int64_t)oc * a.kpad < ((int64_t)1 << 31) &&
+                                 *std::max_element(p.pads, p.pads + 4) <= 2000;
         bool ring = false;  // took the LDS-DMA ring (the only route that reads an upsampled residual)
         if (direct && g.f16 && kh == 3 && kw == 3 && ic == 3 && st == p.strides[1] && (st == 1 || st == 2) &&
             oc <= 32 && a.ldy % 4 == 0 && !getenv("SIMDONNX_HIP_STEM_DIRECT")) {
@@ -1105,9 +1148,10 @@ struct Emitter {
                  {offsetof(sox_igemm_args, add), p.add_value >= 0 ? bind(p.add_value) : none()},
                  {offsetof(sox_igemm_args, y), ybind}, {offsetof(sox_igemm_args, zeros), none()}},
                 (uint32_t)tiles, (uint32_t)((oc + 31) / 32), 1, 256, 0, "conv_halo");
-        } else if (g.f16 && amode == 'v' && !(p.pad_mode == 0 && p.pad_value != 0.0f) &&
-                   (p.pad_mode != 1 || reflect_folds_once(a)) && !getenv("SIMDONNX_HIP_IGEMM")) {
-            // fp16 NHWC with ic % 8 == 0 and zero/reflect padding: the LDS-DMA implicit-GEMM ring
+        } else if (amode == 'v' && !(p.pad_mode == 0 && p.pad_value != 0.0f) &&
+                   (p.pad_mode != 1 || reflect_folds_once(a)) && !getenv("SIMDONNX_HIP_IGEMM") && !f32_short &&
+                   (g.f16 || ring_f32_ok)) {
+            // NHWC rows of whole 16-byte chunks and zero/reflect padding: the LDS-DMA implicit-GEMM ring
             a.res_shift = cov.shift;
             const char* forced = getenv("SIMDONNX_HIP_CONV");
             if (kh == 1 && kw == 1 && st == 1 && p.strides[1] == 1 && !p.pads[0] && !p.pads[1] && !p.pads[2] &&
@@ -1121,8 +1165,7 @@ struct Emitter {
                             p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(),
                             cov.res >= 0 ? bind(cov.res) : p.add_value >= 0 ? bind(p.add_value) : none(), ybind);
             ring = true;
-        } else if (!g.f16 && ic % 16 == 0 && a.k % 64 == 0 && a.k <= 576 && oc % 4 == 0 && a.ldy % 4 == 0 && p.pad_mode == 0 &&
-                   p.pad_value == 0.0f && !getenv("SIMDONNX_HIP_IGEMM")) {
+        } else if (f32_short) {
             // fp32 with a short reduction: the whole 32x32 tile's operands in LDS, K split over the four
             // waves on the fp32 matrix cores, each wave loading its own quarter (conv_f32.hip)
             add(ni, "sox_conv_f32_short_k" + std::to_string(a.k), a,
@@ -1275,7 +1318,7 @@ struct Emitter {
         const bool pad_rows = pad_it != g.padded_ld.end();
         auto ln_it = g.ln_fold.find(ni);
         const bool ln = ln_it != g.ln_fold.end();  // A is a folded LayerNorm's input
-        const bool dma = g.f16 && k % ld() == 0;
+        const bool dma = k % ld() == 0 && (g.f16 || !getenv("SIMDONNX_HIP_IGEMM"));
         if (ln && !dma) fail(SOX_E_INVALID, "Gemm: LayerNorm folded into a Gemm off the LDS-DMA route");
         // opt-in (SIMDONNX_HIP_GEMMPP): whole 256 x 128 tiles, K = 768, bias + none / relu / GELU, at
         // least a tile per CU, on the kernel that runs each tile's epilogue under the next tile's

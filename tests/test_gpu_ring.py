@@ -1,7 +1,7 @@
 """The LDS-DMA ring at the sizes where its tilings, tails and trimmed rings can go wrong, against the
-oracle: K tails (a multiple of 8 that is not one of 64), N that no group of 4 divides, single
+oracle: K tails (a multiple of 8 that is not one of 64; fp32: of 4), N that no group of 4 divides, single
 rows, reductions of one slice up to more than the ring's stages, every tiling the estimate can pick
-(through shapes that pick it), 1x1 convs as dense products.
+(through shapes that pick it), 1x1 convs as dense products, and the fp32 tiles (ring and split K).
 
 Tolerances: 16-bit outputs are one rounding of an fp32 sum (2^-11 / 2^-8 relative to the element, whose
 magnitude is at most the maximum); the fp32 sums of K terms differ in order only, at most K 2^-24 of the sum
@@ -42,7 +42,7 @@ GEMMS = [(1, 8, 1), (1, 64, 64), (3, 16, 5), (64, 24, 64), (47, 40, 88), (65, 72
          (6000, 320, 640), (6016, 328, 1288), (3000, 136, 1000), (4096, 264, 768), (12300, 40, 192), (16640, 200, 384)]
 
 
-@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("case", GEMMS, ids=lambda c: "x".join(map(str, c)))
 def test_gemm_tails_and_tilings(hip, storage, case):
     m, k, n = case
@@ -65,7 +65,7 @@ def test_gemm_tails_and_tilings(hip, storage, case):
 def test_every_default_tiling_is_reached(hip):
     """The shapes above (and the wide products) cover every tiling that the estimate chooses from."""
     kernels = set()
-    for storage in ("f16",):
+    for storage in ("f16", "f32"):
         for m, k, n in GEMMS + [(8192, 768, 3072), (4096, 1024, 2000), (4096, 1024, 1000), (8192, 760, 3000),
                                 (1024, 1536, 1024), (8192, 512, 512), (512, 384, 8192), (8192, 1016, 8192), (8192, 512, 1024)]:
             pb = PlanBuilder()
@@ -75,7 +75,7 @@ def test_every_default_tiling_is_reached(hip):
             g.release()
     want = ["gemm_f16_256x192_w8k64s2", "gemm_f16_256x128_w8k64s2", "gemm_f16_128x64_k64s2e", "gemm_f16_64x64_k64s2",
             "gemm_kt_f16_256x128_w8k64s2", "gemm_kt_f16_64x64_k64s2",
-            "gemm_kt_f16_128x96_k32s2", "gemm_kt_f16_64x64_k32s2"]
+            "gemm_kt_f16_128x96_k32s2", "gemm_kt_f16_64x64_k32s2", "gemm_f32_64x64_k32s2", "conv_f32_split"]
     missing = [w for w in want if "sox_" + w not in kernels]
     assert not missing, (missing, sorted(kernels))
 
@@ -91,7 +91,7 @@ CONVS = [(1, 7, 9, 8, 8, 1, 1, "relu", False, 0), (2, 33, 31, 24, 88, 1, 1, "non
          (1, 1, 5, 8, 9, 3, 1, "none", False, 0), (1, 12, 160, 64, 192, 1, 1, "none", False, 0)]
 
 
-@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("case", CONVS, ids=lambda c: "x".join(map(str, c)))
 def test_conv_tails_and_tilings(hip, storage, case, monkeypatch):
     n, h, w, ic, oc, k, st, act, res, mode = case
