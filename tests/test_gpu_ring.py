@@ -110,3 +110,23 @@ def test_conv_tails_and_tilings(hip, storage, case, monkeypatch):
     assert len(kernels) == 1 and "igemm" not in kernels[0], kernels
     want = O.conv(x, wt, b, r, stride=(st, st), pads=(p, p, p, p), act=act, pad_mode=mode)
     assert max_rel(got, want) < tol(storage, k * k * ic), kernels
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("t", [1, 16, 47, 63])
+def test_fused_block_below_64_rows(hip, storage, t, monkeypatch):
+    """A mixer block of one short line: attention and MLP run fused (the LayerNorms folded for them), within
+    the 16-bit contract of the oracle and of the unfused dispatches."""
+    from oracle.interp import run_plan
+    from test_gpu_workloads import _attention_block_plan
+    plan, x = _attention_block_plan(1, t, seed=143, mlp=True)
+    g = hip.graph(plan, storage)
+    assert [d[0] for d in g.dispatches] == ["qkv_attn", "mlp", "mlp_sum"]
+    g.release()
+    got, _ = run(hip, plan, [x], storage)
+    monkeypatch.setenv("SIMDONNX_HIP_NO_LN_FOLD", "1")
+    unfused, kernels = run(hip, plan, [x], storage)
+    assert len(kernels) > 5
+    want = run_plan(plan, [x], f16_storage="bf16" if storage == "bf16" else True)
+    bound = 5e-3 if storage == "f16" else 2e-2
+    assert max_rel(got, want) < bound and max_rel(got, unfused) < bound
