@@ -469,13 +469,15 @@ typedef struct sox_img2nhwc_args {
 
 /* Image session output (nhwc2img.comp): the ih x iw window at (pt, pl) of NHWC [h][w][3] -> tightly
  * packed u8, byte = clamp(int(v * scale + 0.5), 0, 255); one thread per 4-byte word (3 bpp: words
- * straddle pixels; 4 bpp: one pixel, alpha copied from the uploaded source `alpha`). */
+ * straddle pixels; 4 bpp: one pixel, alpha copied from the uploaded source `alpha`). A launch writes words
+ * [first, nwords); dst may be mapped host memory. */
 typedef struct sox_nhwc2img_args {
     const void* x;
     uint32_t* dst;
     const uint32_t* alpha;
     int32_t h, w, ih, iw, pt, pl, nwords, bpp, swap;
     float scale;
+    int32_t first;
 } sox_nhwc2img_args;
 
 /* Fused transformer MLP (mlp.hip): y = act2(GELU(rstd (x . W1 - mean c1) + b1) . W2 + b2 + res), the

@@ -4033,6 +4033,8 @@ int sox_ctc_argmax(sox_ctc* c, sox_session* s, int32_t feature_value, int32_t ba
 }  // extern "C"
 
 // ---- image session (VkImageSession, Backends/Vulkan/VkImageSession.cs; kernels in tensor.hip) ----
+constexpr uint64_t kImageChunk = 768 << 10;  // bytes: ~14 us of PCIe
+
 struct sox_image_session {
     sox_backend* be = nullptr;
     void* lut = nullptr;  // device [3][256] fp32
@@ -4041,18 +4043,18 @@ struct sox_image_session {
     int pad_multiple = 1;
     sox_graph* g = nullptr;  // the graph of the bound tensor size (reference held by its session)
     sox_session* s = nullptr;
-    void* d_src = nullptr;   // packed u8 pixels, then the 4-byte output words
-    void* d_dst = nullptr;
+    void* d_src = nullptr;    // packed u8 pixels
     uint64_t d_bytes = 0;
-    void* h_stage = nullptr;  // pinned
+    void* h_stage = nullptr;  // pinned and mapped: the pixels on their way up, then the output words
+    std::vector<void*> ev;    // one per output chunk
     uint64_t h_bytes = 0;
 
     ~sox_image_session() {
         if (s) sox_session_destroy(s);
         if (lut) sox_free(lut);
         if (d_src) sox_free(d_src);
-        if (d_dst) sox_free(d_dst);
         if (h_stage) sox_host_free(h_stage);
+        for (void* e : ev) sox_event_destroy(e);
     }
     void pads(int height, int width, int& pt, int& pl, int& h, int& w) const {  // ImageSessionOptions.Pads
         const int ph = (pad_multiple - height % pad_multiple) % pad_multiple;
@@ -4129,12 +4131,10 @@ int sox_image_session_run(sox_image_session* is, sox_graph* graph, const uint8_t
         const uint64_t need = (bytes + 4 + 255) & ~255ull;
         if (need > is->d_bytes) {  // grow-only pixel buffers (a quarter of headroom, VkImageSession.Staging)
             if (is->d_src) sox_free(is->d_src);
-            if (is->d_dst) sox_free(is->d_dst);
-            is->d_src = is->d_dst = nullptr;
+            is->d_src = nullptr;
             is->d_bytes = 0;
             const uint64_t size = need + need / 4;
             check(sox_malloc(&is->d_src, size), "ImageSession pixels");
-            check(sox_malloc(&is->d_dst, size), "ImageSession pixels");
             is->d_bytes = size;
         }
         if (need > is->h_bytes) {
@@ -4146,8 +4146,21 @@ int sox_image_session_run(sox_image_session* is, sox_graph* graph, const uint8_t
             is->h_bytes = size;
         }
         uint8_t* hs = (uint8_t*)is->h_stage;
-        for (int y = 0; y < height; y++) memcpy(hs + (uint64_t)y * row, src + (uint64_t)y * src_stride, row);
-        check(sox_memcpy_h2d(is->d_src, hs, bytes, s->stream), "ImageSession upload");
+        // The frame goes up and comes home in chunks: while one chunk crosses PCIe the host copies the next
+        // between the caller's rows and the staging (a 1920x1080 Bgr24 frame through a six-layer model:
+        // 835 -> 660 us, with the copy up, the copy home and both row copies one after the other before).
+        const int chunks = (int)std::clamp<uint64_t>(bytes / kImageChunk, 1, 8);
+        void* up = graph->be->fn("sox_stage_in_f32");
+        uint64_t sent = 0;  // whole 64-byte lines, the last chunk to the end (the buffers have slack for its last word)
+        for (int c = 0, y = 0; c < chunks; c++) {
+            const int y1 = c + 1 == chunks ? height : (int)((int64_t)height * (c + 1) / chunks);
+            for (; y < y1; y++) memcpy(hs + (uint64_t)y * row, src + (uint64_t)y * src_stride, row);
+            const uint64_t end = c + 1 == chunks ? (bytes + 3) & ~3ull : (uint64_t)y1 * row & ~63ull;
+            const int64_t words = (int64_t)(end - sent) / 4;
+            Staging::launch(up, hs + sent, (uint8_t*)is->d_src + sent, words, std::min<int64_t>(64, (words + 2047) / 2048),
+                            s->stream);
+            sent = end;
+        }
         const bool rgb_bytes = format == SOX_PIX_RGB24 || format == SOX_PIX_RGBA32;
         const int swap = rgb_bytes != is->rgb_order ? 1 : 0;  // ImageSessionOptions.Swap
         const char* ty = graph->bf16 ? "bf16" : graph->f16 ? "f16" : "f32";
@@ -4161,14 +4174,28 @@ int sox_image_session_run(sox_image_session* is, sox_graph* graph, const uint8_t
         sox_nhwc2img_args b{};
         const int64_t nwords = bpp == 4 ? (int64_t)height * width : ((int64_t)height * width * 3 + 3) / 4;
         if (nwords >= ((int64_t)1 << 31)) fail(SOX_E_UNSUPPORTED, "ImageSession.Run: image too large");
-        b.x = s->value_ptr(P.output); b.dst = (uint32_t*)is->d_dst; b.alpha = (const uint32_t*)is->d_src;
-        b.h = h; b.w = w; b.ih = height; b.iw = width; b.pt = pt; b.pl = pl; b.nwords = (int)nwords; b.bpp = bpp;
+        b.x = s->value_ptr(P.output); b.dst = (uint32_t*)hs; b.alpha = (const uint32_t*)is->d_src;
+        b.h = h; b.w = w; b.ih = height; b.iw = width; b.pt = pt; b.pl = pl; b.bpp = bpp;
         b.swap = swap; b.scale = is->scale;
-        const uint32_t g2[3] = {(uint32_t)((nwords + 255) / 256), 1, 1};
-        check(sox_launch(graph->be->fn(std::string("sox_nhwc2img_") + ty), g2, blk, 0, s->stream, &b, sizeof b), "nhwc2img");
-        check(sox_memcpy_d2h(hs, is->d_dst, bytes, s->stream), "ImageSession download");
-        check(sox_stream_sync(s->stream), "ImageSession wait");
-        for (int y = 0; y < height; y++) memcpy(dst + (uint64_t)y * dst_stride, hs + (uint64_t)y * row, row);
+        void* down = graph->be->fn(std::string("sox_nhwc2img_") + ty);
+        while ((int)is->ev.size() < chunks) {
+            void* e = nullptr;
+            check(sox_event_create(&e), "ImageSession event");
+            is->ev.push_back(e);
+        }
+        auto chunk_end = [&](int c) { return c + 1 == chunks ? nwords : nwords * (c + 1) / chunks & ~255ll; };
+        for (int c = 0; c < chunks; c++) {  // straight into the mapped staging
+            b.first = c ? (int)chunk_end(c - 1) : 0;
+            b.nwords = (int)chunk_end(c);
+            const uint32_t g2[3] = {(uint32_t)((b.nwords - b.first + 255) / 256), 1, 1};
+            check(sox_launch(down, g2, blk, 0, s->stream, &b, sizeof b), "nhwc2img");
+            check(sox_event_record(is->ev[c], s->stream), "ImageSession event");
+        }
+        for (int c = 0, y = 0; c < chunks; c++) {
+            check(sox_event_sync(is->ev[c]), "ImageSession wait");
+            const int y1 = c + 1 == chunks ? height : (int)((uint64_t)chunk_end(c) * 4 / row);
+            for (; y < y1; y++) memcpy(dst + (uint64_t)y * dst_stride, hs + (uint64_t)y * row, row);
+        }
     });
 }
 

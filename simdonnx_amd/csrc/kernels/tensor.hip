@@ -618,7 +618,7 @@ extern "C" __global__ void __launch_bounds__(256) sox_img2nhwc_f32(sox_img2nhwc_
 template <typename T>
 __device__ __forceinline__ void nhwc2img_body(const sox_nhwc2img_args& p) {
 #pragma clang fp contract(off)
-    const int w4 = blockIdx.x * blockDim.x + threadIdx.x;
+    const int w4 = p.first + blockIdx.x * blockDim.x + threadIdx.x;
     if (w4 >= p.nwords) return;
     const T* x = (const T*)p.x;
     auto u8 = [&](long i) { return (uint32_t)fminf(fmaxf(to_f(x[i]) * p.scale + 0.5f, 0.0f), 255.0f); };

@@ -70,3 +70,22 @@ def test_image_session_conv_model(hip, fmt, bpp, size, half):
     if bpp == 4:
         assert np.array_equal(out.reshape(height, width, 4)[..., 3], src.reshape(height, width, 4)[..., 3])
     s.close()
+
+
+@pytest.mark.parametrize("fmt,bpp", [("Bgr24", 3), ("Rgba32", 4)])
+@pytest.mark.parametrize("width,height,extra", [(701, 1123, 5), (512, 512, 0), (1201, 1100, 3), (1920, 1080, 0)])
+def test_image_session_frames_of_several_chunks(hip, fmt, bpp, width, height, extra):
+    """Frames that cross PCIe in one to eight chunks whose ends fall inside rows and pixels: a copy model gives
+    back every byte, into another buffer and in place, twice on the same session."""
+    stride = width * bpp + extra
+    src = np.random.default_rng(9).integers(0, 256, (height, stride), dtype=np.uint8)
+    with_pad = HipImageSession(hip, UNIT, pad_multiple=4)
+    th, tw = with_pad.tensor_size(width, height)
+    g = hip.graph(copy_plan(th, tw), True)
+    for _ in range(2):
+        out = with_pad.run(g, src, width, height, fmt)
+        assert np.array_equal(out[:, :width * bpp], src[:, :width * bpp])
+    own = src.copy()
+    with_pad.run(g, own, width, height, fmt, own)
+    assert np.array_equal(own, src)
+    with_pad.close()
