@@ -779,6 +779,7 @@ struct Emitter {
             {"sox_gemm_f16_128x128_k64s2", 128, 128, 64, 2, 0.72f, 0.67f, 4.0f, 1.6f},
             {"sox_gemm_f16_128x64_k64s2e", 128, 64, 64, 2, 0.46f, 0.345f, 3.9f, 0.4f},
             {"sox_gemm_f16_64x64_k64s2", 64, 64, 64, 4, 0.256f, 0.22f, 3.5f, 0.35f},
+            {"sox_gemm_f16_128x32_k64s2", 128, 32, 64, 3, 0.32f, 0.25f, 2.4f, 0.7f},  // n <= 32
             // selectable with SIMDONNX_HIP_GEMM (tuning / tests)
             {"sox_gemm_f16_128x64_k64s2", 128, 64, 64, 3},     {"sox_gemm_f16_64x64_k64s4", 64, 64, 64, 2},
             {"sox_gemm_f16_128x64_k64s4", 128, 64, 64, 1},     {"sox_gemm_f16_256x192_k32s5", 256, 192, 32, 1},
@@ -793,7 +794,8 @@ struct Emitter {
             {"sox_gemm_kt_f16_128x64_k64s2", 128, 64, 64, 3, 0.5f, 0.42f, 3.9f, 0.5f},
             {"sox_gemm_kt_f16_64x64_k64s2", 64, 64, 64, 4, 0.3f, 0.25f, 3.5f, 0.35f},
             {"sox_gemm_kt_f16_128x96_k32s2", 128, 96, 32, 3, 0.3f, 0.26f, 4.0f, 0.7f},
-            {"sox_gemm_kt_f16_64x64_k32s2", 64, 64, 32, 4, 0.19f, 0.16f, 3.4f, 0.35f}};
+            {"sox_gemm_kt_f16_64x64_k32s2", 64, 64, 32, 4, 0.19f, 0.16f, 3.4f, 0.35f},
+            {"sox_gemm_kt_f16_128x32_k32s2", 128, 32, 32, 4, 0.4f, 0.16f, 2.9f, 0.5f}};  // n <= 32
         static const RingCfg cfgs32[] = {
             {"sox_gemm_f32_128x64_k32s2", 128, 64, 32, 3, 1.23f, 1.23f, 4.0f, 1.0f},
             {"sox_gemm_f32_64x64_k32s2", 64, 64, 32, 4, 0.62f, 0.62f, 3.5f, 0.6f},
@@ -801,9 +803,12 @@ struct Emitter {
             {kF32Split, 32, 32, 16, 2, 0.105f, 0.1f, 3.0f, 0.8f}};
         const char* forced = getenv("SIMDONNX_HIP_GEMM");
         const RingCfg* pick;
+        // a 32-wide 16-bit tile only where every wider one is at least half padding: over more columns it reads
+        // A once more per 32 of them (57600 x 72 -> 40: 6.9 us against 64x64's 5.8)
+        const int narrow = a.n <= 32 && !ln ? 1 : 0;
         if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, nullptr, "");
-        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 6, 0, 6, a.m, a.n, a.k, 1, nullptr, "");
-        else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5, a.m, a.n, a.k, 1, forced, "SIMDONNX_HIP_GEMM");
+        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 7, 0, 6 + narrow, a.m, a.n, a.k, 1, nullptr, "");
+        else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5 + narrow, a.m, a.n, a.k, 1, forced, "SIMDONNX_HIP_GEMM");
         a.kpad = pad8(a.k);
         a.lda = a.k;
         a.flags |= SOX_F_DENSE_A;
@@ -850,6 +855,7 @@ struct Emitter {
             {"sox_conv_f16_128x64_k64s2", 128, 64, 64, 3, 0.6f, 0.39f, 4.0f, 0.6f},
             {"sox_conv_f16_64x64_k64s4", 64, 64, 64, 2, 0.42f, 0.29f, 3.8f, 0.4f},
             {"sox_conv_f16_64x64_k32s4", 64, 64, 32, 2, 0.28f, 0.18f, 3.8f, 0.4f},
+            {"sox_conv_f16_128x32_k32s2", 128, 32, 32, 4, 0.38f, 0.22f, 3.8f, 0.4f},  // n <= 32, as the dense one
             // by the rules for large convs below
             {"sox_conv_f16_256x128_w8k64s2", 256, 128, 64, 1}, {"sox_conv_f16_256x256_w8k64s2", 256, 256, 64, 1},
             {"sox_conv_f16_h256", 256, 256, 64, 1}};
@@ -890,7 +896,7 @@ struct Emitter {
             name = "sox_conv_f16_256x128_w8k64s2";
         const int64_t taps = (int64_t)a.kh * a.kw;
         const RingCfg* c =
-            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
+            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 7 : 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
                   : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, nullptr, "");
         if (c->name == kF32Split) {
             launch_f32_split(node, a, x, w, bias, add_b, y, "conv");

@@ -4,6 +4,7 @@
 
 SOX_CONV(sox_conv_bf16_64x64_k32s4, bf16_t, 64, 64, 32, 32, 32, 4, 4, 2, 4)
 SOX_CONV(sox_conv_bf16_64x64_k64s4, bf16_t, 64, 64, 64, 32, 32, 4, 4, 2, 4)
+SOX_CONV(sox_conv_bf16_128x32_k32s2, bf16_t, 128, 32, 32, 32, 32, 2, 4, 4, 4)
 SOX_CONV(sox_conv_bf16_128x64_k64s2, bf16_t, 128, 64, 64, 64, 32, 2, 4, 3, 4)
 SOX_CONV(sox_conv_bf16_128x96_k32s2, bf16_t, 128, 96, 32, 32, 96, 2, 4, 3, 4)
 SOX_CONV(sox_conv_bf16_128x96_k64s2, bf16_t, 128, 96, 64, 32, 96, 2, 4, 2, 4)

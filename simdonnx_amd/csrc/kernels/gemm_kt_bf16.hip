@@ -7,3 +7,4 @@ SOX_GEMM_KT(sox_gemm_kt_bf16_128x64_k64s2, bf16_t, 128, 64, 64, 64, 32, 2, 4, 3,
 SOX_GEMM_KT(sox_gemm_kt_bf16_64x64_k64s2, bf16_t, 64, 64, 64, 32, 32, 2, 4, 4, 4, false)
 SOX_GEMM_KT(sox_gemm_kt_bf16_128x96_k32s2, bf16_t, 128, 96, 32, 32, 96, 2, 4, 3, 4, false)
 SOX_GEMM_KT(sox_gemm_kt_bf16_64x64_k32s2, bf16_t, 64, 64, 32, 32, 32, 2, 4, 4, 4, false)
+SOX_GEMM_KT(sox_gemm_kt_bf16_128x32_k32s2, bf16_t, 128, 32, 32, 32, 32, 2, 4, 4, 4, true)

@@ -39,7 +39,8 @@ def run(hip, plan, ins, storage):
 
 GEMMS = [(1, 8, 1), (1, 64, 64), (3, 16, 5), (64, 24, 64), (47, 40, 88), (65, 72, 97), (33, 120, 6), (130, 200, 200),
          (256, 1000, 96), (200, 520, 190), (40, 192, 768), (63, 768, 192), (786, 760, 760), (900, 16, 300), (2000, 24, 96),
-         (6000, 320, 640), (6016, 328, 1288), (3000, 136, 1000), (4096, 264, 768), (12300, 40, 192), (16640, 200, 384)]
+         (6000, 320, 640), (6016, 328, 1288), (3000, 136, 1000), (4096, 264, 768), (12300, 40, 192), (16640, 200, 384),
+         (33000, 16, 7), (65537, 72, 24), (66000, 64, 32), (40001, 128, 17)]
 
 
 @pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
@@ -75,7 +76,8 @@ def test_every_default_tiling_is_reached(hip):
             g.release()
     want = ["gemm_f16_256x192_w8k64s2", "gemm_f16_256x128_w8k64s2", "gemm_f16_128x64_k64s2e", "gemm_f16_64x64_k64s2",
             "gemm_kt_f16_256x128_w8k64s2", "gemm_kt_f16_64x64_k64s2",
-            "gemm_kt_f16_128x96_k32s2", "gemm_kt_f16_64x64_k32s2", "gemm_f32_64x64_k32s2", "conv_f32_split"]
+            "gemm_kt_f16_128x96_k32s2", "gemm_f16_128x32_k64s2", "gemm_kt_f16_128x32_k32s2",
+            "gemm_kt_f16_64x64_k32s2", "gemm_f32_64x64_k32s2", "conv_f32_split"]
     missing = [w for w in want if "sox_" + w not in kernels]
     assert not missing, (missing, sorted(kernels))
 
@@ -88,7 +90,9 @@ CONVS = [(1, 7, 9, 8, 8, 1, 1, "relu", False, 0), (2, 33, 31, 24, 88, 1, 1, "non
          (1, 40, 40, 64, 24, 5, 1, "relu", False, 0), (2, 40, 40, 128, 256, 3, 1, "gelu", False, 0),
          (1, 31, 33, 96, 96, 3, 1, "relu", False, 1), (8, 50, 30, 48, 56, 5, 1, "none", False, 0),
          (4, 64, 64, 40, 80, 3, 1, "relu", False, 0), (8, 64, 64, 128, 128, 3, 1, "relu", False, 0),
-         (1, 1, 5, 8, 9, 3, 1, "none", False, 0), (1, 12, 160, 64, 192, 1, 1, "none", False, 0)]
+         (1, 1, 5, 8, 9, 3, 1, "none", False, 0), (1, 12, 160, 64, 192, 1, 1, "none", False, 0),
+         (1, 301, 299, 24, 32, 3, 2, "relu", False, 0), (1, 250, 203, 16, 20, 3, 1, "none", True, 0),
+         (2, 160, 240, 40, 7, 5, 1, "relu", False, 1)]
 
 
 @pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
