@@ -1148,12 +1148,21 @@ struct Emitter {
             // 3x3 stride 1 with few output channels: every tap from one LDS copy of the input halo
             // (at stride 2 a pixel feeds ~2 outputs per tap row and the implicit-GEMM ring is faster)
             const int tiles = ((cow + 15) / 16) * ((coh + 7) / 8) * nb;
-            add(ni, "sox_conv_halo_f16_3x3s1", a,
+            // whole 16-byte output chunks and up to 32 input channels: persistent workgroups with the filter in
+            // registers (1x544x960 32 -> 32 45.5 -> 22.0 us, 1x480x480 16 -> 16 19.3 -> 8.9, 1x60x60 32 -> 32
+            // 5.8 -> 4.5). Up to 64: its 36 fragments take ~3 us to fetch, so from three tiles a CU on
+            // (1x544x960 64 -> 64 109 -> 61 us, 8x128x128 48 -> 48 28.2 -> 16.7; at 1.8 a CU, 8x56x56 64 -> 64,
+            // 12.6 against the LDS filter's 9.0). Three or two workgroups fit a CU; with two blocks of output
+            // channels the grid is two high (32 -> 64 over 544x960: 36.6 us, 39.7 with three a CU and block).
+            const int64_t cus = std::max(1, g.be->info.compute_units), nblk = (oc + 31) / 32;
+            const bool reg = (ic <= 32 || (ic <= 64 && tiles * nblk >= 3 * cus)) && ((oc | a.ldy) & 7) == 0 && ybind.offset % 16 == 0;
+            const uint32_t grid = reg ? (uint32_t)(std::min<int64_t>(tiles, cus * (ic <= 32 ? 3 : 2) / nblk) + 7) / 8 * 8 : (uint32_t)tiles;
+            add(ni, !reg ? "sox_conv_halo_f16_3x3s1" : ic <= 32 ? "sox_conv_halo_f16_3x3s1_c32" : "sox_conv_halo_f16_3x3s1_c64", a,
                 {{offsetof(sox_igemm_args, x), xb}, {offsetof(sox_igemm_args, w), wb},
                  {offsetof(sox_igemm_args, bias), p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none()},
                  {offsetof(sox_igemm_args, add), p.add_value >= 0 ? bind(p.add_value) : none()},
                  {offsetof(sox_igemm_args, y), ybind}, {offsetof(sox_igemm_args, zeros), none()}},
-                (uint32_t)tiles, (uint32_t)((oc + 31) / 32), 1, 256, 0, "conv_halo");
+                grid, (uint32_t)nblk, 1, 256, 0, "conv_halo");
         } else if (amode == 'v' && !(p.pad_mode == 0 && p.pad_value != 0.0f) &&
                    (p.pad_mode != 1 || reflect_folds_once(a)) && !getenv("SIMDONNX_HIP_IGEMM") && !f32_short &&
                    (g.f16 || ring_f32_ok)) {

@@ -175,3 +175,185 @@ SOX_HALO(sox_conv_halo_f16_3x3s1, half_t, 3, 3, 1, 1, 2, false)
 SOX_HALO(sox_conv_halo_bf16_3x3s1, bf16_t, 3, 3, 1, 1, 2, false)
 SOX_HALO(sox_conv_halo_f16_3x3s1_upcat, half_t, 3, 3, 1, 1, 2, true)
 SOX_HALO(sox_conv_halo_bf16_3x3s1_upcat, bf16_t, 3, 3, 1, 1, 2, true)
+
+// 3x3 stride-1 convs over at most 32 or 64 input channels (sox_conv_halo_*_3x3s1_c32 / _c64, whole 16-byte
+// output chunks): persistent workgroups, the filter in registers.
+//  * The kernel above copies 23 KB of weights, and the zeros of an absent second channel block, into LDS for
+//    every 128 pixels. Here a wave keeps the 18 weight fragments a block of 32 input channels has for its 32
+//    output channels (72 registers a block) and walks over tiles of 8 x 16 pixels; only input halos cross the
+//    LDS, one block ahead of the multiply.
+//  * A halo pixel is 64 bytes (4 chunks of 8 channels), its chunks XOR-swizzled by pixel so that 16 consecutive
+//    pixels fall on 16 distinct 16-byte bank groups: two stages are 24 KB and several workgroups share a CU.
+//  * Each XCD takes a contiguous band of tiles, so the pixels that neighbouring halos share come from its L2.
+//  * Stores: a permlane32 swap of accumulator pairs gives each lane 8 consecutive channels (16 bytes).
+template <typename T, int NCB> __device__ __forceinline__ void halo_reg_body(const sox_igemm_args& p) {
+    typedef vec_t<T, 8> T8;
+    typedef vec_t<T, 4> T4;
+    constexpr int TW = 16, TH = 8, HW = TW + 2, HH = TH + 2, HP = HH * HW, IT = (HP * 4 + 255) / 256;
+    constexpr int STAGE = IT * 256 * 16;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem0[STAGE], smem1[STAGE];
+    __shared__ float sbias[32];
+
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l32 = lane & 31, hl = lane >> 5;
+    const int N = p.n, n0 = blockIdx.y * 32;
+    const int tiles_x = (p.ow + TW - 1) / TW, tiles_y = (p.oh + TH - 1) / TH;
+    const int tiles = tiles_x * tiles_y * (int)(p.m / ((long)p.oh * p.ow));
+    // the grid is a multiple of 8 and workgroups go to the 8 XCDs in turn
+    const int xcd = blockIdx.x & 7, band = (tiles + 7) / 8, step = gridDim.x >> 3;
+    const int last = min(tiles, (xcd + 1) * band);
+    int tile = xcd * band + (blockIdx.x >> 3);
+    if (tile >= last) return;
+    const T* __restrict__ X = (const T*)p.x;
+    const T* __restrict__ Z = (const T*)p.zeros;
+
+    int hoff[IT], hy[IT], hx[IT], hc[IT];  // this thread's DMA slots: offset from the halo's first pixel, row, column, channel
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+        const int q = i * 256 + t, hp = q >> 2, sub = (q & 3) ^ ((hp >> 2) & 3);
+        hy[i] = hp / HW;
+        hx[i] = hp - hy[i] * HW;
+        hc[i] = sub * 8;
+        hoff[i] = (hy[i] * p.iw + hx[i]) * p.ic + hc[i];
+        if (q >= HP * 4) hy[i] = 1 << 30;  // outside every image: zeros
+    }
+    auto issue = [&](int tl, int c0, unsigned char* stage) __attribute__((always_inline)) {
+        const int tx = tl % tiles_x, tyb = tl / tiles_x, ty = tyb % tiles_y, b = tyb / tiles_y;
+        const int iy0 = ty * TH - p.pt, ix0 = tx * TW - p.pl;
+        const T* src0 = X + (((long)b * p.ih + iy0) * p.iw + ix0) * p.ic + c0;
+        unsigned char* st = stage + wave * 64 * 16;
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            const bool ok = (unsigned)(iy0 + hy[i]) < (unsigned)p.ih && (unsigned)(ix0 + hx[i]) < (unsigned)p.iw &&
+                            c0 + hc[i] < p.ic;
+            const T* src = ok ? src0 + hoff[i] : Z;
+            __builtin_amdgcn_global_load_lds(src, LDS_PTR(st + i * 256 * 16), 16, 0, 0);
+        }
+    };
+    issue(tile, 0, smem0);
+
+    // weight fragments: row n0 + l32, channels 32 block + 16 s + 8 hl ..+7 of each tap
+    T8 wf[NCB * 18];
+    static_for<0, NCB * 18>([&](auto ts) {
+        constexpr int cb = decltype(ts)::value / 18, tap = decltype(ts)::value % 18 / 2, s = decltype(ts)::value % 2;
+        const int c = cb * 32 + s * 16 + hl * 8;
+        const T* src = n0 + l32 < N && c < p.ic ? (const T*)p.w + (long)(n0 + l32) * p.kpad + tap * p.ic + c : Z;
+        wf[decltype(ts)::value] = *(const T8*)src;
+    });
+    const bool has_bias = (p.flags & SOX_F_BIAS) != 0;
+    if (t < 32) sbias[t] = has_bias && n0 + t < N ? p.bias[n0 + t] : 0.0f;  // published by the first barrier
+    const int py = 2 * wave + (l32 >> 4), px = l32 & 15;
+    int a_off[9];
+    static_for<0, 9>([&](auto tt) {
+        constexpr int tap = decltype(tt)::value;
+        const int hp = (py + tap / 3) * HW + px + tap % 3;
+        a_off[tap] = (hp * 4 + (hl ^ ((hp >> 2) & 3))) * 16;
+    });
+    const int act = (p.flags & SOX_F_ACT_MASK) >> SOX_F_ACT_SHIFT;
+    const T* __restrict__ R = (p.flags & SOX_F_RESIDUAL) ? (const T*)p.add : nullptr;
+
+    wait_lgkmcnt0();
+    float16v acc;
+    // multiplies channel block cb of the tile from st while the block (next_tile, next_cb) loads into next
+    auto block = [&](auto cbc, const unsigned char* st, unsigned char* next, int next_tile, int next_cb) __attribute__((always_inline)) {
+        constexpr int cb = decltype(cbc)::value;
+        wait_vmcnt<0>();               // this wave's part of the halo landed
+        __builtin_amdgcn_s_barrier();  // ... and every wave's; the other stage has been read
+        if (next_tile < last) issue(next_tile, next_cb * 32, next);
+        if constexpr (cb == 0)
+            static_for<0, 4>([&](auto qq) {
+                constexpr int q = decltype(qq)::value;
+                const float4v b4 = *(const float4v*)(sbias + 8 * q + 4 * hl);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[4 * q + e] = b4[e];
+            });
+        // a row of taps' pixels is read while the row before multiplies
+        auto taps = [&](auto steps) __attribute__((always_inline)) {
+            constexpr int S = decltype(steps)::value;  // 16-channel steps
+            T8 af[2][3 * S];
+            auto read = [&](auto yy) __attribute__((always_inline)) {
+                constexpr int ky = decltype(yy)::value;
+                static_for<0, 3 * S>([&](auto xs) {
+                    constexpr int kx = decltype(xs)::value / S, s = decltype(xs)::value % S;
+                    af[ky & 1][kx * S + s] = *(const T8*)(st + (a_off[ky * 3 + kx] ^ (32 * s)));
+                });
+            };
+            read(std::integral_constant<int, 0>());
+            static_for<0, 3>([&](auto yy) {
+                constexpr int ky = decltype(yy)::value;
+                if constexpr (ky < 2) read(std::integral_constant<int, ky + 1>());
+                static_for<0, 3 * S>([&](auto xs) {
+                    constexpr int kx = decltype(xs)::value / S, s = decltype(xs)::value % S;
+                    acc = mfma32x32x16(wf[cb * 18 + 2 * (ky * 3 + kx) + s], af[ky & 1][kx * S + s], acc);
+                });
+            });
+        };
+        if (cb < NCB - 1 || p.ic > cb * 32 + 16) taps(std::integral_constant<int, 2>());
+        else taps(std::integral_constant<int, 1>());
+        wait_lgkmcnt0();
+    };
+    auto store = [&]() __attribute__((always_inline)) {
+        const int tx = tile % tiles_x, tyb = tile / tiles_x, ty = tyb % tiles_y, b = tyb / tiles_y;
+        const int oy = ty * TH + py, ox = tx * TW + px;
+        const bool in = oy < p.oh && ox < p.ow;
+        const long row = (((long)b * p.oh + oy) * p.ow + ox) * p.ldy;
+        T* __restrict__ Y = (T*)p.y + row;
+        if (R && in)
+            static_for<0, 4>([&](auto qq) {
+                constexpr int q = decltype(qq)::value;
+                const int n = n0 + 8 * q + 4 * hl;
+                const T4 r = *(const T4*)(n < N ? R + row + n : Z);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[4 * q + e] += (float)r[e];
+            });
+        T4 h[4];
+        auto finish = [&](auto ac) __attribute__((always_inline)) {
+            static_for<0, 16>([&](auto qe) {
+                constexpr int i = decltype(qe)::value;
+                h[i / 4][i % 4] = (T)out_act<T, decltype(ac)::value>(acc[i], act);
+            });
+        };
+        switch (act) {
+            case SOX_ACT_NONE: finish(std::integral_constant<int, SOX_ACT_NONE>()); break;
+            case SOX_ACT_RELU: finish(std::integral_constant<int, SOX_ACT_RELU>()); break;
+            case SOX_ACT_HARDSWISH: finish(std::integral_constant<int, SOX_ACT_HARDSWISH>()); break;
+            default: finish(std::integral_constant<int, -1>());
+        }
+        static_for<0, 2>([&](auto pp) {  // lanes 0..31 take channels 16 P ..+7, lanes 32..63 16 P + 8 ..+15
+            constexpr int P = decltype(pp)::value;
+            union { T4 v; unsigned u[2]; } lo, hi;
+            union { T8 v; unsigned u[4]; } o;
+            lo.v = h[2 * P];
+            hi.v = h[2 * P + 1];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(lo.u[k], hi.u[k], false, false);
+                o.u[k] = sw[0];
+                o.u[2 + k] = sw[1];
+            }
+            const int n = n0 + 16 * P + 8 * hl;
+            if (in && n < N) *(T8*)(Y + n) = o.v;
+        });
+    };
+    // two arrays, not one of two stages: the compiler then sees that the reads of one do not touch the other's
+    // DMA, and waits for none of it
+    constexpr std::integral_constant<int, 0> c0;
+    while (true) {
+        if constexpr (NCB == 2) {
+            block(c0, smem0, smem1, tile, 1);
+            block(std::integral_constant<int, 1>(), smem1, smem0, tile + step, 0);
+            store();
+        } else {
+            block(c0, smem0, smem1, tile + step, 0);
+            store();
+            if ((tile += step) >= last) break;
+            block(c0, smem1, smem0, tile + step, 0);
+            store();
+        }
+        if ((tile += step) >= last) break;
+    }
+}
+
+extern "C" __global__ void __launch_bounds__(256, 3) sox_conv_halo_f16_3x3s1_c32(sox_igemm_args p) { halo_reg_body<half_t, 1>(p); }
+extern "C" __global__ void __launch_bounds__(256, 3) sox_conv_halo_bf16_3x3s1_c32(sox_igemm_args p) { halo_reg_body<bf16_t, 1>(p); }
+extern "C" __global__ void __launch_bounds__(256, 2) sox_conv_halo_f16_3x3s1_c64(sox_igemm_args p) { halo_reg_body<half_t, 2>(p); }
+extern "C" __global__ void __launch_bounds__(256, 2) sox_conv_halo_bf16_3x3s1_c64(sox_igemm_args p) { halo_reg_body<bf16_t, 2>(p); }

@@ -134,3 +134,33 @@ def test_fused_block_below_64_rows(hip, storage, t, monkeypatch):
     want = run_plan(plan, [x], f16_storage="bf16" if storage == "bf16" else True)
     bound = 5e-3 if storage == "f16" else 2e-2
     assert max_rel(got, want) < bound and max_rel(got, unfused) < bound
+
+
+# (batch, h, w, ic, oc, act, residual, concat): both register kernels and the LDS one, tile edges, a last channel
+# block of 8 .. 32 channels, one and two blocks of output channels, fewer tiles than XCDs, several tiles a workgroup
+HALOS = [(1, 8, 16, 8, 8, "relu", False, False), (1, 9, 17, 32, 40, "hardswish", True, False), (3, 50, 70, 24, 64, "gelu", False, True),
+         (1, 1, 1, 16, 16, "none", True, False), (2, 300, 310, 16, 24, "none", True, False), (1, 200, 333, 32, 64, "none", False, False),
+         (1, 260, 270, 40, 64, "relu", True, False), (2, 250, 200, 64, 32, "hardswish", False, False),
+         (1, 320, 330, 56, 24, "none", False, True), (1, 40, 40, 64, 32, "relu", False, False), (1, 21, 33, 32, 12, "none", False, False)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("case", HALOS, ids=lambda c: "x".join(str(v) for v in c))
+def test_halo_filter_in_registers(hip, storage, case):
+    n, h, w, ic, oc, act, res, cat = case
+    x = stored(synth.normal(144, 1, (n, h, w, ic), 1.0), storage)
+    wt = stored(synth.normal(144, 2, (oc, ic, 3, 3), (9 * ic)**-0.5), storage)
+    b = synth.uniform(144, 3, (oc,), -0.5, 0.5)
+    r = stored(synth.normal(144, 4, (n, h, w, oc), 1.0), storage)
+    pb = PlanBuilder()
+    ins = [pb.input((n, ic, h, w), NHWC, "x")] + ([pb.input((n, oc, h, w), NHWC, "r")] if res else [])
+    y = pb.conv(ins[0], wt, b, stride=1, pad=1, act=act, add=ins[1] if res else None, name="conv")
+    if cat:  # the second half of a concat
+        y = pb.concat_channels([pb.conv(ins[0], wt, b, stride=1, pad=1, name="first"), y])
+    got, kernels = run(hip, pb.build(y), [x] + ([r] if res else []), storage)
+    tiles = n * -(-h // 8) * -(-w // 16) * -(-oc // 32)
+    want_k = "3x3s1" if oc % 8 or (ic > 32 and tiles < 768) else "3x3s1_c32" if ic <= 32 else "3x3s1_c64"
+    assert kernels[-1] == f"sox_conv_halo_{storage}_{want_k}", kernels
+    want = O.conv(x, wt, b, r if res else None, stride=(1, 1), pads=(1, 1, 1, 1), act=act)
+    if cat: want = np.concatenate([O.conv(x, wt, b, None, stride=(1, 1), pads=(1, 1, 1, 1), act="none"), want], axis=-1)
+    assert max_rel(got, want) < tol(storage, 9 * ic), kernels
