@@ -54,3 +54,27 @@ def test_unit_runner_waves_match_sessions(hip, half):
             ref = run_plan(plans[i], [xs[i]], f16_storage=half)
             assert max_rel(got, ref) < (2e-2 if half else 1e-4)
     r.close()
+
+
+@pytest.mark.parametrize("streams,units,cut", [(1, 9, 4), (2, 8, 0), (3, 10, 7), (4, 6, 1), (5, 13, 6)])
+def test_unit_runner_enqueues_from_two_threads(hip, streams, units, cut):
+    """Enough launches for the second enqueuing thread (and one stream, which never takes it): every unit gives
+    the bits of its session over several submits with new inputs, whatever the streams and waves."""
+    graphs = [hip.graph(line_plan(64 + 32 * i), True) for i in range(units)]
+    r = HipUnitRunner(hip, streams=streams)
+    for i, g in enumerate(graphs):
+        r.add(g)
+        if cut and i + 1 == cut:
+            r.cut()
+    assert sum(len(g.kernels) + 2 for g in graphs) >= 24
+    for run in range(3):
+        xs = [synth.normal(73 + run, i, (1, 32, 64 + 32 * i, 3), 1.0) for i in range(units)]
+        for i, x in enumerate(xs):
+            r.input(i)[:] = x.reshape(-1)
+        r.submit()
+        r.wait()
+        for i, (g, x) in enumerate(zip(graphs, xs)):
+            with HipInferenceSession(g) as s:
+                s.set_input(x)
+                assert np.array_equal(r.output(i), s.run()), (run, i)
+    r.close()
