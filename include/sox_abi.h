@@ -259,6 +259,14 @@ typedef struct sox_cvt_args {
     int64_t count;
 } sox_cvt_args;
 
+/* Rows of c elements copied with each padded with zeros to cp (a multiple of 16 bytes). */
+typedef struct sox_padc_args {
+    const void* x;
+    void* y;
+    int64_t rows;
+    int32_t c, cp;
+} sox_padc_args;
+
 /* LayerNorm over the innermost dim, one wave per row (layernorm.comp; Kernels/Ops.cs:544-574). */
 typedef struct sox_ln_args {
     const void* x;

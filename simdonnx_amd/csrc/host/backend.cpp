@@ -333,14 +333,20 @@ enum { CK_CONVT_NK = 9 };  // ConvTranspose weights [IC][OC][KH][KW] as a GEMM B
 // nb of 32 columns, k-step s, lane l -> 8 values W[16 s + 8 (l / 32) + e][32 nb + l % 32], e = 0..7, at
 // ((nb * K / 16 + s) * 64 + l) * 8 + e, so a wave's fragment load is one contiguous KiB
 enum { CK_FRAG32 = 10 };
+// conv weights over channels padded with zeros to a multiple of 8 or 4 (16-byte chunks of 16-bit or fp32):
+// [OC][tap * ICp + ic], ICp = ceil(IC / pad) pad
+enum { CK_CONVWT_P8 = 11, CK_CONVWT_P4 = 12 };
 
 int pad8(int k) { return (k + 7) & ~7; }
+int round_up(int k, int to) { return (k + to - 1) / to * to; }
 
 // Element count of a const in a packing (Extensions.cs:144-159; K rows padded to 8 for 16-byte loads).
 int64_t packed_elems(const PlanValue& v, int kind) {
     const auto& s = v.shape;
     switch (kind) {
         case SOX_CK_CONVWT: return (int64_t)s[0] * pad8(s[1] * s[2] * s[3]);
+        case CK_CONVWT_P8: case CK_CONVWT_P4:
+            return (int64_t)s[0] * pad8(s[2] * s[3] * round_up(s[1], kind == CK_CONVWT_P8 ? 8 : 4));
         case SOX_CK_GEMMNK: return (int64_t)s[1] * pad8(s[0]);
         case CK_GEMMNK_T: return (int64_t)s[0] * pad8(s[1]);
         case CK_CONVT_NK: return (int64_t)s[1] * s[2] * s[3] * pad8(s[0]);
@@ -361,6 +367,13 @@ void pack_const(const PlanValue& v, int kind, float* d) {
             for (int o = 0; o < oc; o++)
                 for (int c = 0; c < ic; c++)
                     for (int t = 0; t < taps; t++) d[(int64_t)o * kp + t * ic + c] = src[((int64_t)o * ic + c) * taps + t];
+            break;
+        }
+        case CK_CONVWT_P8: case CK_CONVWT_P4: {
+            const int oc = s[0], ic = s[1], taps = s[2] * s[3], icp = round_up(ic, kind == CK_CONVWT_P8 ? 8 : 4), kp = pad8(taps * icp);
+            for (int o = 0; o < oc; o++)
+                for (int c = 0; c < ic; c++)
+                    for (int t = 0; t < taps; t++) d[(int64_t)o * kp + t * icp + c] = src[((int64_t)o * ic + c) * taps + t];
             break;
         }
         case CK_FRAG32: {  // [K][N] -> fragment order (see CK_FRAG32)
@@ -436,6 +449,9 @@ int64_t axis_stride(const PlanValue& v, int axis);
 // ---------------------------------------------------------------------------------------------
 // Lowering of one ExecNode (the analogue of VkGraphModel.Emit, VkGraph.cs:472-1112).
 // ---------------------------------------------------------------------------------------------
+bool conv_pads_channels(const sox_graph& g, const PlanNode& n);
+bool gemm_pads_k(const sox_graph& g, int64_t m, int n, int k);
+
 struct Emitter {
     sox_graph& g;
     std::set<int> skip;  // nodes already lowered into a previous node's dispatch
@@ -647,6 +663,16 @@ struct Emitter {
     sox_bind scratch(uint64_t bytes) {
         g.scratch_bytes = std::max<uint64_t>(g.scratch_bytes, (bytes + 255) & ~255ull);
         return sox_bind{SOX_SLOT_ARENA, 0, g.scratch_off, bytes};
+    }
+
+    // rows x c elements of x copied to scratch with each row padded with zeros to cp
+    sox_bind pad_channels(int node, sox_bind x, int64_t rows, int c, int cp) {
+        const sox_bind y = scratch((uint64_t)rows * cp * g.es);
+        sox_padc_args a{};
+        a.rows = rows; a.c = c; a.cp = cp;
+        add(node, std::string("sox_padc_") + (g.f16 ? "b16" : "b32"), a,
+            {{offsetof(sox_padc_args, x), x}, {offsetof(sox_padc_args, y), y}}, blocks(rows * (cp / ld())), 1, 1, 256, 0, "pad_channels");
+        return y;
     }
 
     template <class A>
@@ -1033,7 +1059,7 @@ struct Emitter {
             return;
         }
         // an SE gate folded into this conv: read the gate's input with the gated weight copy
-        sox_bind xb = bind(n.in[0]), wb = bind(n.in[1], SOX_CK_CONVWT);
+        sox_bind xb = bind(n.in[0]), wb = conv_pads_channels(g, n) ? none() : bind(n.in[1], SOX_CK_CONVWT);
         auto fold_it = se_fold.find(ni);
         if (fold_it != se_fold.end()) {
             xb = bind(fold_it->second.first);
@@ -1091,6 +1117,15 @@ struct Emitter {
         a.lda = 0;
         char amode = ic % ld() == 0 ? 'v' : 's';
         const int st = p.strides[0];
+        if (fold_it == se_fold.end() && conv_pads_channels(g, n)) {
+            const int icp = round_up(ic, ld());
+            xb = pad_channels(ni, xb, (int64_t)nb * ih * iw, ic, icp);
+            wb = bind(n.in[1], kh * kw == 1 ? SOX_CK_CONVWT : g.f16 ? CK_CONVWT_P8 : CK_CONVWT_P4);
+            a.ic = ic = icp;
+            a.k = kh * kw * ic;
+            a.kpad = pad8(a.k);
+            amode = 'v';
+        }
         // fp32 with a short reduction (conv_f32.hip)
         const bool f32_short = !g.f16 && ic % 16 == 0 && a.k % 64 == 0 && a.k <= 576 && oc % 4 == 0 && a.ldy % 4 == 0 &&
                                p.pad_mode == 0 && p.pad_value == 0.0f && !getenv("SIMDONNX_HIP_IGEMM");
@@ -1336,7 +1371,8 @@ struct Emitter {
         const bool pad_rows = pad_it != g.padded_ld.end();
         auto ln_it = g.ln_fold.find(ni);
         const bool ln = ln_it != g.ln_fold.end();  // A is a folded LayerNorm's input
-        const bool dma = k % ld() == 0 && (g.f16 || !getenv("SIMDONNX_HIP_IGEMM"));
+        const bool pad_k = gemm_pads_k(g, m, nn, k);
+        const bool dma = pad_k || (k % ld() == 0 && (g.f16 || !getenv("SIMDONNX_HIP_IGEMM")));
         if (ln && !dma) fail(SOX_E_INVALID, "Gemm: LayerNorm folded into a Gemm off the LDS-DMA route");
         // opt-in (SIMDONNX_HIP_GEMMPP): whole 256 x 128 tiles, K = 768, bias + none / relu / GELU, at
         // least a tile per CU, on the kernel that runs each tile's epilogue under the next tile's
@@ -1366,11 +1402,12 @@ struct Emitter {
         }
         if (dma) {
             sox_igemm_args a{};
-            a.m = (int)m; a.n = nn; a.k = k;
+            a.m = (int)m; a.n = nn; a.k = pad_k ? round_up(k, ld()) : k;
             a.flags = (p.bias_value >= 0 ? SOX_F_BIAS : 0) | (act << SOX_F_ACT_SHIFT) |
                       (residual >= 0 ? SOX_F_RESIDUAL : 0) | (pad_rows ? SOX_F_PAD_ROWS : 0);
             a.ldy = pad_rows ? pad_it->second : nn;
-            launch_gemm_dma(ni, a, bind(n.in[0]), bind(n.in[1], p.trans_b ? CK_GEMMNK_T : SOX_CK_GEMMNK),
+            const sox_bind xb = pad_k ? pad_channels(ni, bind(n.in[0]), m, k, a.k) : bind(n.in[0]);
+            launch_gemm_dma(ni, a, xb, bind(n.in[1], p.trans_b ? CK_GEMMNK_T : SOX_CK_GEMMNK),
                             p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(), res_b, bind(out_value),
                             ln ? &ln_it->second : nullptr, ln ? "gemm_ln" : "gemm");
             return;
@@ -2918,6 +2955,38 @@ void plan_upsample_add(sox_graph& g) {
     }
 }
 
+// Rows that are not whole 16-byte chunks (channels, or a Gemm's K, no multiple of 8; fp32: of 4) cannot take the
+// LDS-DMA kernels: padded with zeros into scratch first, they can, for one pass over the input. Against the
+// implicit GEMM's element gather, fp16 / fp32: Gemm 4096 x 1023 -> 2000 172 -> 37 / 350 -> 218 us, 256 x 1001 -> 97
+// 73 -> 13.6 / 41 -> 12.2, 64 x 65 -> 64 10.2 -> 5.3 / 6.6 -> 5.7; conv 4x128x128 65 -> 129 3x3 190 -> 90 / 309 -> 245,
+// 1x20x20 250 -> 250 3x3 (fp32 251) 156 -> 22 / 89 -> 21, 1x32x32 33 -> 64 3x3 27 -> 8.9 / 15 -> 8.2. Not where few
+// channels are mostly padding (the ring multiplies whole 32- or 16-channel slices of every tap: 1x224x224 3 -> 64
+// 7x7 16.4 us, 20.5 padded; fp32 1x480x480 5 -> 9 3x3 50 / 67), nor a short fp32 K (5000 x 30 -> 90 7.2 / 7.6),
+// nor where the copy would grow the arena by more than kPadBytes.
+constexpr int64_t kPadBytes = 1ll << 30;
+bool pads_rows(const sox_graph& g, int64_t rows, int c, int64_t n, int taps) {
+    const int ld = g.f16 ? 8 : 4;
+    return c % ld != 0 && c >= (taps > 1 ? 9 : g.f16 ? 16 : 32) && !getenv("SIMDONNX_HIP_IGEMM") &&
+           rows * round_up(c, ld) * (g.f16 ? 2 : 4) <= kPadBytes && n * pad8(taps * round_up(c, ld)) < ((int64_t)1 << 31);
+}
+bool gemm_pads_k(const sox_graph& g, int64_t m, int n, int k) { return pads_rows(g, m, k, n, 1); }
+bool conv_pads_channels(const sox_graph& g, const PlanNode& n) {
+    const auto& p = n.p<sox_conv_p>();
+    const int ld = g.f16 ? 8 : 4;
+    const PlanValue& wv = g.V(n.in[1]);
+    const std::vector<int> xs = g.V(n.in[0]).phys(), ys = g.V(n.out[0]).phys();
+    if (p.group != 1 || p.has_pool || xs.size() != 4 || ys.size() != 4 || wv.shape.size() != 4) return false;
+    sox_igemm_args a{};
+    a.kh = p.kernel[0]; a.kw = p.kernel[1]; a.sh = p.strides[0]; a.sw = p.strides[1]; a.pt = p.pads[0]; a.pl = p.pads[1];
+    a.ih = xs[1]; a.iw = xs[2]; a.oh = ys[1]; a.ow = ys[2];
+    const int oc = wv.shape[0], ic = xs[3], taps = a.kh * a.kw;
+    if (oc % ld == 0 && taps * ic <= 64 && oc <= 128) return false;  // the direct convs read such rows themselves
+    if (p.pad_mode == 0 ? p.pad_value != 0.0f : !Emitter::reflect_folds_once(a)) return false;
+    // what the ring's packed origins hold
+    if (a.ih > 30000 || a.iw > 30000 || *std::max_element(p.pads, p.pads + 4) > 2000) return false;
+    return pads_rows(g, (int64_t)xs[0] * a.ih * a.iw, ic, oc, taps);
+}
+
 // Const kinds each node's dispatches bind (the per-consumer packing, VkGraph.cs:81-143).
 void collect_consts(sox_graph& g, std::vector<std::pair<int, int>>& need) {
     auto want = [&](int v, int k) {
@@ -2931,7 +3000,9 @@ void collect_consts(sox_graph& g, std::vector<std::pair<int, int>>& need) {
             case SOX_OP_CONV: {
                 const auto& p = n.p<sox_conv_p>();
                 want(n.in[0], SOX_CK_RAW);
-                want(n.in[1], p.group > 1 ? SOX_CK_DWW : SOX_CK_CONVWT);
+                want(n.in[1], p.group > 1 ? SOX_CK_DWW
+                              : p.kernel[0] * p.kernel[1] > 1 && conv_pads_channels(g, n) ? (g.f16 ? CK_CONVWT_P8 : CK_CONVWT_P4)
+                                                                                          : SOX_CK_CONVWT);
                 want(p.bias_value, SOX_CK_F32);
                 want(p.add_value, SOX_CK_RAW);
                 break;

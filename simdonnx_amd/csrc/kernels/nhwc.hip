@@ -1973,3 +1973,26 @@ extern "C" __global__ void __launch_bounds__(256) sox_conv_direct_333_pool_f32(s
 extern "C" __global__ void __launch_bounds__(256) sox_conv_direct_pool_f16(sox_igemm_args p) { conv_direct_body<half_t, 8, true>(p); }
 extern "C" __global__ void __launch_bounds__(256) sox_conv_direct_pool_bf16(sox_igemm_args p) { conv_direct_body<bf16_t, 8, true>(p); }
 extern "C" __global__ void __launch_bounds__(256) sox_conv_direct_pool_f32(sox_igemm_args p) { conv_direct_body<float, 4, true>(p); }
+
+// ------------------------------------------------------------------------------------------
+// Rows of c elements to rows of cp, a multiple of 16 bytes, with zeros behind them: what the LDS-DMA kernels
+// read where a tensor's own rows are not whole 16-byte chunks. One chunk per thread: the source is aligned to
+// an element only, so its loads are element by element, served by L1 after the first
+// (4096 x 1023 to 1024 in fp16: ~8 us).
+template <typename U>
+__device__ __forceinline__ void padc_body(const sox_padc_args& p) {
+    typedef vec_t<U, 16 / sizeof(U)> V;
+    constexpr int E = 16 / sizeof(U);
+    const int cpr = p.cp / E;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.rows * cpr) return;
+    const long row = i / cpr;
+    const int c0 = (int)(i - row * cpr) * E;
+    const U* x = (const U*)p.x + row * p.c;
+    V v;
+#pragma unroll
+    for (int e = 0; e < E; e++) v[e] = c0 + e < p.c ? x[c0 + e] : (U)0;
+    ((V*)p.y)[i] = v;
+}
+extern "C" __global__ void __launch_bounds__(256) sox_padc_b16(sox_padc_args p) { padc_body<unsigned short>(p); }
+extern "C" __global__ void __launch_bounds__(256) sox_padc_b32(sox_padc_args p) { padc_body<unsigned int>(p); }

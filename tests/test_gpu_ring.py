@@ -164,3 +164,47 @@ def test_halo_filter_in_registers(hip, storage, case):
     want = O.conv(x, wt, b, r if res else None, stride=(1, 1), pads=(1, 1, 1, 1), act=act)
     if cat: want = np.concatenate([O.conv(x, wt, b, None, stride=(1, 1), pads=(1, 1, 1, 1), act="none"), want], axis=-1)
     assert max_rel(got, want) < tol(storage, 9 * ic), kernels
+
+
+ODD_GEMMS = [(1, 9, 1), (5, 17, 3), (64, 65, 64), (33, 33, 130), (130, 1001, 97), (700, 255, 255), (2000, 30, 90), (3000, 127, 20)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", ODD_GEMMS, ids=lambda c: "x".join(map(str, c)))
+def test_gemm_rows_padded_to_chunks(hip, storage, case):
+    """K that is no whole 16-byte chunk: the rows are padded into scratch first, from `short` on."""
+    m, k, n = case
+    x = stored(synth.normal(145, 1, (m, k), 1.0), storage)
+    w = stored(synth.normal(145, 2, (k, n), k**-0.5), storage)
+    b = synth.uniform(145, 3, (n,), -0.5, 0.5)
+    pb = PlanBuilder()
+    got, kernels = run(hip, pb.build(pb.gemm(pb.input((m, k), None, "x"), w, b, act="gelu", name="gemm")), [x], storage)
+    short, ld = (32, 4) if storage == "f32" else (16, 8)
+    assert ("padc" in kernels[0]) == (k >= short and k % ld != 0), kernels
+    assert max_rel(got, O.gemm(x, w, b, act="gelu")) < tol(storage, k), kernels
+
+
+ODD_CONVS = [(1, 7, 9, 9, 5, 3, 1, "relu", False, 0), (2, 16, 16, 17, 17, 3, 1, "none", True, 0), (1, 40, 30, 33, 64, 3, 2, "gelu", False, 0),
+             (1, 25, 31, 129, 60, 1, 1, "relu", True, 0), (2, 50, 40, 31, 45, 5, 1, "hardswish", False, 1),
+             (1, 20, 20, 250, 250, 3, 1, "none", False, 0), (1, 60, 60, 11, 3, 3, 1, "relu", False, 0), (1, 30, 30, 7, 20, 3, 1, "none", False, 0),
+             (1, 33, 20, 50, 41, 1, 2, "none", False, 0)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", ODD_CONVS, ids=lambda c: "x".join(map(str, c)))
+def test_conv_channels_padded_to_chunks(hip, storage, case):
+    n, h, w, ic, oc, k, st, act, res, mode = case
+    p = k // 2
+    oh, ow = (h + 2 * p - k) // st + 1, (w + 2 * p - k) // st + 1
+    x = stored(synth.normal(146, 1, (n, h, w, ic), 1.0), storage)
+    wt = stored(synth.normal(146, 2, (oc, ic, k, k), (k * k * ic)**-0.5), storage)
+    b = synth.uniform(146, 3, (oc,), -0.5, 0.5)
+    r = stored(synth.normal(146, 4, (n, oh, ow, oc), 1.0), storage) if res else None
+    pb = PlanBuilder()
+    ins = [pb.input((n, ic, h, w), NHWC, "x")] + ([pb.input((n, oc, oh, ow), NHWC, "r")] if res else [])
+    y = pb.conv(ins[0], wt, b, stride=st, pad=p, act=act, add=ins[1] if res else None, pad_mode=mode, name="conv")
+    got, kernels = run(hip, pb.build(y), [x] + ([r] if res else []), storage)
+    ld = 4 if storage == "f32" else 8
+    assert ("padc" in kernels[0]) == (ic % ld != 0 and ic >= 9), kernels
+    want = O.conv(x, wt, b, r, stride=(st, st), pads=(p, p, p, p), act=act, pad_mode=mode)
+    assert max_rel(got, want) < tol(storage, k * k * ic), kernels
