@@ -187,7 +187,7 @@ def test_gemm_rows_padded_to_chunks(hip, storage, case):
 ODD_CONVS = [(1, 7, 9, 9, 5, 3, 1, "relu", False, 0), (2, 16, 16, 17, 17, 3, 1, "none", True, 0), (1, 40, 30, 33, 64, 3, 2, "gelu", False, 0),
              (1, 25, 31, 129, 60, 1, 1, "relu", True, 0), (2, 50, 40, 31, 45, 5, 1, "hardswish", False, 1),
              (1, 20, 20, 250, 250, 3, 1, "none", False, 0), (1, 60, 60, 11, 3, 3, 1, "relu", False, 0), (1, 30, 30, 7, 20, 3, 1, "none", False, 0),
-             (1, 33, 20, 50, 41, 1, 2, "none", False, 0)]
+             (1, 33, 20, 50, 41, 1, 2, "none", False, 0), (1, 20, 20, 63, 64, 3, 1, "relu", False, 0), (2, 10, 13, 15, 16, 3, 1, "none", True, 0)]
 
 
 @pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
