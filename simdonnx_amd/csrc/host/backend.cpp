@@ -1374,13 +1374,13 @@ struct Emitter {
         const bool pad_k = gemm_pads_k(g, m, nn, k);
         const bool dma = pad_k || (k % ld() == 0 && (g.f16 || !getenv("SIMDONNX_HIP_IGEMM")));
         if (ln && !dma) fail(SOX_E_INVALID, "Gemm: LayerNorm folded into a Gemm off the LDS-DMA route");
-        // opt-in (SIMDONNX_HIP_GEMMPP): whole 256 x 128 tiles, K = 768, bias + none / relu / GELU, at
+        // opt-in (SIMDONNX_HIP_GEMMPP), 16-bit graphs: whole 256 x 128 tiles, K = 768, bias + none / relu / GELU, at
         // least a tile per CU, on the kernel that runs each tile's epilogue under the next tile's
         // matrix-core work (gemm_pp.h; measured slower than the ring on the 8192 x 768 x 3072 Gemm)
         const char* forced_gemm = getenv("SIMDONNX_HIP_GEMM");
         const char* want_pp = getenv("SIMDONNX_HIP_GEMMPP");
         const int cus_pp = std::max(1, g.be->info.compute_units);
-        if (dma && !ln && residual < 0 && !pad_rows && !(forced_gemm && *forced_gemm) &&
+        if (g.f16 && dma && !ln && residual < 0 && !pad_rows && !(forced_gemm && *forced_gemm) &&
             want_pp && *want_pp && strcmp(want_pp, "0") != 0 && m % 256 == 0 && nn % 128 == 0 && k == 768 &&
             (act == SOX_ACT_NONE || act == SOX_ACT_RELU || act == SOX_ACT_GELU) &&
             (m / 256) * (int64_t)(nn / 128) >= cus_pp) {

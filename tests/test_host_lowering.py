@@ -238,3 +238,22 @@ def test_large_conv_tile_takes_inputs_under_2_pow_31_elements(offline, monkeypat
     monkeypatch.setenv("SIMDONNX_HIP_CONV", "sox_conv_f16_256x256_w8k64s2")
     with pytest.raises(N.NotSupportedError):
         offline.graph(big, "f16")
+
+
+def test_gemm_pp_takes_16_bit_graphs_only(offline, monkeypatch):
+    """SIMDONNX_HIP_GEMMPP opts 16-bit Gemms of whole 256x128 tiles with K = 768 into sox_gemmpp_*, whose kernels
+    read 16-bit operands: the same fp32 Gemm stays on the fp32 kernels."""
+    import numpy as np
+    from simdonnx_amd.plan import PlanBuilder
+    monkeypatch.setenv("SIMDONNX_HIP_GEMMPP", "1")
+    pb = PlanBuilder()
+    y = pb.gemm(pb.input((8192, 768), None, "a"), np.zeros((768, 1024), np.float32), None, act="gelu", name="gemm")
+    plan = pb.build(y)
+    for storage in STORAGES:
+        g = offline.graph(plan, storage)
+        kernels = g.kernels
+        g.release()
+        if storage == "f32":
+            assert all("gemmpp" not in k and "f32" in k for k in kernels), kernels
+        else:
+            assert kernels == [f"sox_gemmpp_{storage}_256x128_k768_gelu"], kernels
