@@ -2536,7 +2536,8 @@ bool fusable_mlp(sox_graph& g, int f1, int x, sox_graph::Mlp& f);
 // pass of sums and sums of squares, as the reference's GPU LayerNorm takes them
 // (Backends/Vulkan/Shaders/layernorm.comp:24-38). Taken only where the Gemm runs on the LDS-DMA
 // ring (K % 64 == 0, N % 4 == 0 or padded rows; at least 64 rows, or fewer where the Gemm then runs in
-// a fused attention or MLP) and no node in between writes over the LayerNorm's input; the Gemm's output moves to a buffer of its own when the arena plan put it
+// a fused attention or MLP), gamma W keeps the storage type's precision and no node in between writes over
+// the LayerNorm's input; the Gemm's output moves to a buffer of its own when the arena plan put it
 // over that input (dead after the LayerNorm, read by the Gemm now).
 void fold_layernorm_into_gemm(sox_graph& g) {
     if (!g.f16 || getenv("SIMDONNX_HIP_NO_LN_FOLD")) return;
@@ -2581,15 +2582,27 @@ void fold_layernorm_into_gemm(sox_graph& g) {
         if (xv.count() / K < 64 && fusable_attention(g, gi, x) < 0 && !fusable_mlp(g, gi, x, probe)) continue;
         PlanValue w2 = wv, b2, c2;
         w2.name = wv.name + ".ln";
-        std::vector<double> bsum(N, 0.0), csum(N, 0.0);
+        std::vector<double> bsum(N, 0.0), csum(N, 0.0), wsq(N, 0.0), esq(N, 0.0);
+        bool finite = true;
         for (int k = 0; k < K; k++)
             for (int n = 0; n < N; n++) {
                 const size_t at = gp.trans_b ? (size_t)n * K + k : (size_t)k * N + n;
                 const float w = wv.floats[at];
                 w2.floats[at] = w * gv.floats[k];
                 bsum[n] += (double)bv.floats[k] * w;
-                csum[n] += g.round16(w2.floats[at]);
+                const double v = w2.floats[at], stored = g.round16(w2.floats[at]);
+                csum[n] += stored;
+                wsq[n] += v * v;
+                if (!g.bf16 && std::fabs(v) < 0x1p-14) esq[n] += (stored - v) * (stored - v);
+                finite = finite && std::isfinite(stored);
             }
+        // gamma W has to fit fp16 as W does: finite, and what a column's values below the normal range lose stays
+        // under what rounding takes from the others (0.15 of half a unit in the last place, squared). Weights of
+        // 0.02 under gamma 1e-3, 16 rows of 192: 9.3e-4 from 64 bits folded, 3.7e-4 as two nodes (gamma 3e-3 4.3e-4 and
+        // 3.6e-4, gamma 1e-2 3.6e-4 both, gamma 1 3.0e-4 and 3.7e-4).
+        bool keeps = finite;
+        for (int n = 0; n < N; n++) keeps = keeps && esq[n] <= 0.15 * 0x1p-22 * wsq[n];
+        if (!keeps) continue;
         b2.is_const = c2.is_const = true;
         b2.shape = c2.shape = {N};
         b2.name = wv.name + ".ln_bias";

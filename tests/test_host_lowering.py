@@ -257,3 +257,25 @@ def test_gemm_pp_takes_16_bit_graphs_only(offline, monkeypatch):
             assert all("gemmpp" not in k and "f32" in k for k in kernels), kernels
         else:
             assert kernels == [f"sox_gemmpp_{storage}_256x128_k768_gelu"], kernels
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("rows", [16, 128])
+@pytest.mark.parametrize("gamma", [1.0, 1e-2, 3e-3, 1e-3, 4e6])
+def test_layernorm_folds_where_its_weights_keep_their_precision(offline, gamma, rows, storage):
+    """LayerNorm -> fc1 + GELU -> fc2 folds the gamma into fc1's weights. With weights of 0.02, gamma 3e-3 or 1e-3 takes
+    most of them below fp16's normal range and 4e6 past its largest value: such a LayerNorm stays a node of its own
+    (bf16 has fp32's range and folds)."""
+    import numpy as np
+    from simdonnx_amd import synth
+    from simdonnx_amd.plan import PlanBuilder
+    pb = PlanBuilder()
+    x = pb.input((1, rows, 192), None, "x")
+    h = pb.layer_norm(x, np.full(192, gamma, np.float32), np.zeros(192, np.float32), 1e-6, name="ln")
+    h = pb.gemm(h, synth.normal(5, 1, (192, 768), 0.02), np.zeros(768, np.float32), act="gelu", name="fc1")
+    y = pb.gemm(h, synth.normal(5, 2, (768, 192), 0.02), np.zeros(192, np.float32), name="fc2")
+    g = offline.graph(pb.build(y), storage)
+    labels = [d[0] for d in g.dispatches]
+    g.release()
+    folds = storage == "bf16" or gamma in (1.0, 1e-2)
+    assert labels[0] == ("mlp" if folds else "layernorm"), labels
