@@ -120,8 +120,7 @@ def build_libs(verbose=False):
     cxx = os.path.join(ROCM, "llvm", "bin", "clang++")
     if not os.path.exists(cxx):
         cxx = _hipcc()
-    # -mf16c: const packing rounds weights to fp16 (a library call per value without it)
-    common = ["-O2", "-mf16c", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include", "-Wall",
+    common = ["-O2", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include", "-Wall",
               "-Wno-unused-result"]
     thin = os.path.join(LIB, "libsoxhip.so")
     # the static device scratch (sox_scratch.hip) is the one host-library source compiled as HIP: its
@@ -168,7 +167,7 @@ def build_sanitized_backend(verbose=False):
     kernel choice) of every workload plan on a backend created without a device
     (tests/test_host_lowering.py)."""
     os.makedirs(SAN_DIR, exist_ok=True)
-    _run([_host_cxx(), "-O1", "-g", "-mf16c", "-fno-omit-frame-pointer", *SAN_FLAGS, "-fPIC", "-std=c++17", "-Wall",
+    _run([_host_cxx(), "-O1", "-g", "-fno-omit-frame-pointer", *SAN_FLAGS, "-fPIC", "-std=c++17", "-Wall",
           "-Wno-unused-result", f"-I{BUILD}", "-shared", "-o", SAN_BACKEND, os.path.join(HDIR, "backend.cpp"),
           os.path.join(BUILD, "resources.S"), f"-L{LIB}", "-lsoxhip", "-Wl,-rpath,$ORIGIN/../../lib",
           f"-Wl,-rpath,{ROCM}/lib"])

@@ -111,3 +111,14 @@ def test_kernels_use_no_scratch():
                 spills[name] = private
     assert count > 50
     assert not spills, spills
+
+
+def test_host_libraries_build_for_any_cpu(monkeypatch):
+    """The host libraries are compiled without machine options: CPU extensions are asked for at run time, in
+    functions of their own."""
+    from simdonnx_amd import build as B
+    cmds = []
+    monkeypatch.setattr(B, "_run", lambda cmd: cmds.append(cmd))
+    B.build_libs()
+    assert len(cmds) >= 3
+    assert not [a for c in cmds for a in c if a.startswith("-m")], cmds
