@@ -3017,11 +3017,13 @@ void plan_upsample_add(sox_graph& g) {
 // 1x20x20 250 -> 250 3x3 (fp32 251) 156 -> 22 / 89 -> 21, 1x32x32 33 -> 64 3x3 27 -> 8.9 / 15 -> 8.2. Not where few
 // channels are mostly padding (the ring multiplies whole 32- or 16-channel slices of every tap: 1x224x224 3 -> 64
 // 7x7 16.4 us, 20.5 padded; fp32 1x480x480 5 -> 9 3x3 50 / 67), nor a short fp32 K (5000 x 30 -> 90 7.2 / 7.6),
-// nor where the copy would grow the arena by more than kPadBytes.
+// nor where the copy would grow the arena by more than kPadBytes. SIMDONNX_HIP_NO_PAD_ROWS leaves every such row
+// to the implicit GEMM, for an arena without the copies.
 constexpr int64_t kPadBytes = 1ll << 30;
 bool pads_rows(const sox_graph& g, int64_t rows, int c, int64_t n, int taps) {
     const int ld = g.f16 ? 8 : 4;
     return c % ld != 0 && c >= (taps > 1 ? 9 : g.f16 ? 16 : 32) && !getenv("SIMDONNX_HIP_IGEMM") &&
+           !getenv("SIMDONNX_HIP_NO_PAD_ROWS") &&
            rows * round_up(c, ld) * (g.f16 ? 2 : 4) <= kPadBytes && n * pad8(taps * round_up(c, ld)) < ((int64_t)1 << 31);
 }
 bool gemm_pads_k(const sox_graph& g, int64_t m, int n, int k) { return pads_rows(g, m, k, n, 1); }

@@ -279,3 +279,30 @@ def test_layernorm_folds_where_its_weights_keep_their_precision(offline, gamma, 
     g.release()
     folds = storage == "bf16" or gamma in (1.0, 1e-2)
     assert labels[0] == ("mlp" if folds else "layernorm"), labels
+
+
+@pytest.mark.parametrize("storage", STORAGES)
+def test_padded_rows_can_be_refused(offline, storage, monkeypatch):
+    """Rows of odd channel counts are copied to padded ones in the arena; SIMDONNX_HIP_NO_PAD_ROWS keeps the arena
+    to the plan's activations and leaves the other kernels as they are."""
+    import numpy as np
+    from simdonnx_amd.plan import NHWC, PlanBuilder
+    pb = PlanBuilder()
+    x = pb.input((1, 65, 128, 128), NHWC, "x")
+    h = pb.conv(x, np.zeros((129, 65, 3, 3), np.float32), np.zeros(129, np.float32), pad=1, name="odd")
+    y = pb.conv(h, np.zeros((64, 129, 1, 1), np.float32), np.zeros(64, np.float32), name="odd1")
+    y = pb.conv(y, np.zeros((64, 64, 1, 1), np.float32), np.zeros(64, np.float32), name="even")
+    plan = pb.build(y)
+    g = offline.graph(plan, storage)
+    kernels, arena = g.kernels, g.arena_bytes
+    _check_binds(g)
+    g.release()
+    monkeypatch.setenv("SIMDONNX_HIP_NO_PAD_ROWS", "1")
+    g = offline.graph(plan, storage)
+    plain, plain_arena = g.kernels, g.arena_bytes
+    _check_binds(g)
+    g.release()
+    assert sum("padc" in k for k in kernels) == 2 and not any("padc" in k for k in plain)
+    assert plain[-1] == kernels[-1] and ["igemm" in k for k in plain] == [True, True, False], plain
+    es = 4 if storage == "f32" else 2
+    assert plain_arena <= (plan.arena_floats * es + 255) // 256 * 256 < arena
