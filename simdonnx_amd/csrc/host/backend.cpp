@@ -915,6 +915,7 @@ struct Emitter {
                          sox_bind y) {
         static const RingCfg cfgs16[] = {
             {"sox_conv_f16_128x128_k64s2", 128, 128, 64, 2, 1.0f, 0.72f, 4.5f, 1.2f},
+            {"sox_conv_f16_128x128_k32s4", 128, 128, 32, 2, 0.5f, 0.46f, 3.5f, 2.0f},
             {"sox_conv_f16_128x96_k64s2", 128, 96, 64, 2, 0.8f, 0.57f, 4.2f, 0.8f},
             {"sox_conv_f16_128x96_k32s2", 128, 96, 32, 3, 0.5f, 0.365f, 4.2f, 0.8f},
             {"sox_conv_f16_128x64_k64s2", 128, 64, 64, 3, 0.6f, 0.39f, 4.0f, 0.6f},
@@ -961,7 +962,7 @@ struct Emitter {
             name = "sox_conv_f16_256x128_w8k64s2";
         const int64_t taps = (int64_t)a.kh * a.kw;
         const RingCfg* c =
-            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 7 : 6, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
+            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 8 : 7, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
                   : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, nullptr, "");
         if (c->name == kF32Split) {
             launch_f32_split(node, a, x, w, bias, add_b, y, "conv");

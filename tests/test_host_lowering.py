@@ -306,3 +306,25 @@ def test_padded_rows_can_be_refused(offline, storage, monkeypatch):
     assert plain[-1] == kernels[-1] and ["igemm" in k for k in plain] == [True, True, False], plain
     es = 4 if storage == "f32" else 2
     assert plain_arena <= (plan.arena_floats * es + 255) // 256 * 256 < arena
+
+
+def _conv_kernel(offline, storage, n, h, w, ic, oc, k, stride):
+    import numpy as np
+    from simdonnx_amd.plan import NHWC, PlanBuilder
+    pb = PlanBuilder()
+    x = pb.input((n, ic, h, w), NHWC, "x")
+    y = pb.conv(x, np.zeros((oc, ic, k, k), np.float32), np.zeros(oc, np.float32), stride=stride, pad=k // 2, name="c")
+    g = offline.graph(pb.build(y), storage)
+    kernels = g.kernels
+    g.release()
+    assert len(kernels) == 1, kernels
+    return kernels[0]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+def test_many_taps_of_few_channels_take_the_wide_shallow_tile(offline, storage):
+    """5x5 convs over at most 32 channels of large maps: 128x128 tiles with 32-deep slices, 40 us where the 64x64 tile
+    takes 55; few channels on small maps stay on the small tiles."""
+    for ic in (8, 24, 32):
+        assert _conv_kernel(offline, storage, 8, 93, 91, ic, 112, 5, 1) == f"sox_conv_{storage}_128x128_k32s4"
+        assert _conv_kernel(offline, storage, 1, 20, 20, ic, 112, 5, 1) == f"sox_conv_{storage}_64x64_k32s4"
