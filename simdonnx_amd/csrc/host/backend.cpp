@@ -810,10 +810,17 @@ struct Emitter {
         const int64_t cus = std::max(1, g.be->info.compute_units);
         return (uint32_t)std::min<int64_t>(c.tiles(m, n), cus * c.wgs_per_cu);
     }
+    // Rows that are not whole 4-element groups leave the ring as single elements, 32 rows an instruction, at a rate
+    // that no tiling changes: 2.5 us per million (20000 x 8 -> 1142 fp16: 74 us, aligned 1440 25). The split tile's
+    // lanes lie along a row: 0.7.
+    static float ragged_us(const RingCfg& c, int64_t m, int64_t n) {
+        return (c.name == kF32Split ? 0.7e-6f : 2.5e-6f) * (float)(m * n);
+    }
     // The tiling of an m x n product over `taps` taps of k reduction elements each: the forced one, else the
-    // one of [first, last) with the smallest estimate
+    // one of [first, last) with the smallest estimate (est, where the caller wants it)
     const RingCfg& ring_pick(const RingCfg* cfgs, size_t ncfg, int first, int last, int64_t m, int64_t n, int64_t k, int64_t taps,
-                             const char* forced, const char* what) const {
+                             bool ragged, const char* forced, const char* what, float* est = nullptr) const {
+        if (est) *est = 0.0f;
         if (forced && *forced) {
             for (size_t i = 0; i < ncfg; i++)
                 if (!strcmp(cfgs[i].name, forced)) return cfgs[i];
@@ -825,19 +832,52 @@ struct Emitter {
         for (int i = first; i < last; i++) {
             const RingCfg& c = cfgs[i];
             const float q = (float)((c.tiles(m, n) + cus - 1) / cus), nk = (float)(taps * ((k + c.bk - 1) / c.bk));
-            const float t = c.base + q * c.tile + nk * std::max(c.lat, q * c.thr);
+            const float t = c.base + q * c.tile + nk * std::max(c.lat, q * c.thr) + (ragged ? ragged_us(c, m, n) : 0.0f);
             if (i == first || t < best) {
                 pick = i;
                 best = t;
             }
         }
+        if (est) *est = best;
         return cfgs[pick];
+    }
+
+    // Whether the implicit GEMM (igemm.hip) beats a ring estimate of ring_us over k reduction elements in all. It stores
+    // single elements of 16 adjacent columns at 1.5 us per million whatever the row length, and it packs the taps of
+    // few channels into one reduction where the ring multiplies a slice of mostly zeros for each. Its estimate has the
+    // ring's form, fits over 5000 random products and fp32 convs, each timed on every kernel; it has to win by a
+    // tenth. On those the pick is within 1% of the fastest kernel on average (ring only: 3 to 5%). Ring only / now:
+    // fp16 20000 x 16 -> 1142 74 / 35 us, 8000 x 24 -> 301 10.1 / 6.7; fp32 8000 x 16 -> 1142 41.7 / 21.6,
+    // conv 4x250x16 8 -> 344 3x3 39.4 / 25.6, 1x128x277 4 -> 366 5x5 3.1 times. 16-bit products only with ragged rows
+    // and from 2^19 outputs on: below, its small tiles lose (22 x 8 -> 168 6.5 us, ring 2.9).
+    bool igemm_wins(float ring_us, int64_t m, int n, int64_t k, char amode, bool ragged) {
+        if (ring_us <= 0.0f || getenv("SIMDONNX_HIP_RING")) return false;  // (a forced tiling; tests of the ring)
+        if (g.f16 && !(ragged && m * n >= 1 << 19)) return false;
+        struct Cost { const char* tile; int bk; float lat, thr, base, tile_us, ragged; };
+        static const Cost costs[] = {
+            {"f32_32x32_d", 64, 0.92f, 0.52f, 2.3f, 0.11f, 0.7f},  {"f32_64x64_d", 32, 1.26f, 0.76f, 3.7f, 0.88f, 0.0f},
+            {"f32_32x32_v", 64, 1.06f, 0.62f, 2.5f, 0.7f, 0.9f},  {"f32_64x64_v", 32, 1.36f, 0.85f, 4.9f, 0.76f, 0.0f},
+            {"16_64x32_d", 32, 0.43f, 0.14f, 2.5f, 0.31f, 2.1f},   {"16_64x32_dk", 128, 0.69f, 0.53f, 3.1f, 0.0f, 1.2f},
+            {"16_64x64_d", 32, 0.1f, 0.21f, 4.6f, 0.38f, 0.1f},    {"16_64x64_dk", 128, 0.93f, 0.79f, 3.3f, 1.4f, 0.7f},
+            {"16_128x128_d", 32, 0.34f, 0.54f, 2.0f, 5.0f, 0.0f}};
+        int bm, bn;
+        const std::string kernel = igemm_kernel(m, n, (int)k, amode, bm, bn);
+        const int64_t cus = std::max(1, g.be->info.compute_units);
+        for (const Cost& c : costs) {
+            const size_t at = kernel.rfind(c.tile);
+            if (at == std::string::npos || at + strlen(c.tile) != kernel.size()) continue;
+            const float q = (float)((((m + bm - 1) / bm) * ((n + bn - 1) / bn) + cus - 1) / cus), nk = (float)((k + c.bk - 1) / c.bk);
+            const float t = c.base + q * c.tile_us + nk * std::max(c.lat, q * c.thr) + (ragged ? c.ragged * 1e-6f * (float)(m * n) : 0.0f);
+            return 1.1f * t < ring_us;
+        }
+        return false;
     }
 
     // Dense product on the LDS-DMA ring (gemm_ring.h): a Gemm, or a 1x1 conv over its pixels. a holds m, n, k
     // (whole 16-byte chunks: a multiple of 8, fp32 of 4), ldy and the epilogue flags.
+    // igemm: the implicit GEMM's mode for these operands where it may take the product instead, else 0.
     void launch_gemm_dma(int node, sox_igemm_args a, sox_bind x, sox_bind w, sox_bind bias, sox_bind add_b, sox_bind y,
-                         const sox_graph::LnFold* ln, const std::string& label) {
+                         const sox_graph::LnFold* ln, const std::string& label, char igemm) {
         static const RingCfg cfgs16[] = {
             {"sox_gemm_f16_256x192_w8k64s2", 256, 192, 64, 1, 1.6f, 1.6f, 4.0f, 2.0f},
             {"sox_gemm_f16_256x128_w8k64s2", 256, 128, 64, 1, 1.3f, 1.3f, 3.3f, 2.0f},
@@ -871,9 +911,20 @@ struct Emitter {
         // a 32-wide 16-bit tile only where every wider one is at least half padding: over more columns it reads
         // A once more per 32 of them (57600 x 72 -> 40: 6.9 us against 64x64's 5.8)
         const int narrow = a.n <= 32 && !ln ? 1 : 0;
-        if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, nullptr, "");
-        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 7, 0, 6 + narrow, a.m, a.n, a.k, 1, nullptr, "");
-        else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5 + narrow, a.m, a.n, a.k, 1, forced, "SIMDONNX_HIP_GEMM");
+        const bool ragged = ((a.flags & SOX_F_PAD_ROWS) ? a.ldy : a.ldy | a.n) % 4 != 0;
+        float est;
+        if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, ragged, nullptr, "", &est);
+        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 7, 0, 6 + narrow, a.m, a.n, a.k, 1, ragged, nullptr, "", &est);
+        else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5 + narrow, a.m, a.n, a.k, 1, ragged, forced, "SIMDONNX_HIP_GEMM", &est);
+        if (igemm && igemm_wins(est, a.m, a.n, a.k, igemm, ragged)) {
+            if (igemm == 'd') {
+                a.kpad = pad8(a.k);
+                a.lda = a.k;
+                a.flags |= SOX_F_DENSE_A;
+            }
+            launch_igemm(node, a, x, w, bias, add_b, y, igemm, label);
+            return;
+        }
         a.kpad = pad8(a.k);
         a.lda = a.k;
         a.flags |= SOX_F_DENSE_A;
@@ -961,9 +1012,15 @@ struct Emitter {
             // large convs: at least two rounds of 256x128 tiles on every CU, 8 waves each
             name = "sox_conv_f16_256x128_w8k64s2";
         const int64_t taps = (int64_t)a.kh * a.kw;
+        const bool ragged = !(a.flags & SOX_F_CONVT) && (a.ldy | a.n) % 4 != 0;
+        float est = 0.0f;
         const RingCfg* c =
-            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 8 : 7, a.m, a.n, a.ic, taps, name, "SIMDONNX_HIP_CONV")
-                  : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, nullptr, "");
+            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 8 : 7, a.m, a.n, a.ic, taps, ragged, name, "SIMDONNX_HIP_CONV")
+                  : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, ragged, nullptr, "", &est);
+        if (!g.f16 && igemm_wins(est, a.m, a.n, a.k, 'v', ragged)) {
+            launch_igemm(node, a, x, w, bias, add_b, y, 'v', "conv");
+            return;
+        }
         if (c->name == kF32Split) {
             launch_f32_split(node, a, x, w, bias, add_b, y, "conv");
             return;
@@ -1249,7 +1306,7 @@ struct Emitter {
                 !(forced && *forced)) {
                 // a 1x1 conv over its pixels is a dense product: no receptive fields to address
                 launch_gemm_dma(ni, a, xb, wb, p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(),
-                                p.add_value >= 0 ? bind(p.add_value) : none(), ybind, nullptr, "conv");
+                                p.add_value >= 0 ? bind(p.add_value) : none(), ybind, nullptr, "conv", g.f16 ? 0 : 'v');
             } else
             launch_conv_dma(ni, a, xb, wb,
                             p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(),
@@ -1446,7 +1503,7 @@ struct Emitter {
             const sox_bind xb = pad_k ? pad_channels(ni, bind(n.in[0]), m, k, a.k) : bind(n.in[0]);
             launch_gemm_dma(ni, a, xb, bind(n.in[1], p.trans_b ? CK_GEMMNK_T : SOX_CK_GEMMNK),
                             p.bias_value >= 0 ? bind(p.bias_value, SOX_CK_F32) : none(), res_b, bind(out_value),
-                            ln ? &ln_it->second : nullptr, ln ? "gemm_ln" : "gemm");
+                            ln ? &ln_it->second : nullptr, ln ? "gemm_ln" : "gemm", ln || pad_rows || pad_k ? 0 : 'd');
             return;
         }
         char amode;

@@ -328,3 +328,35 @@ def test_many_taps_of_few_channels_take_the_wide_shallow_tile(offline, storage):
     for ic in (8, 24, 32):
         assert _conv_kernel(offline, storage, 8, 93, 91, ic, 112, 5, 1) == f"sox_conv_{storage}_128x128_k32s4"
         assert _conv_kernel(offline, storage, 1, 20, 20, ic, 112, 5, 1) == f"sox_conv_{storage}_64x64_k32s4"
+
+
+def _gemm_kernel(offline, storage, m, k, n):
+    import numpy as np
+    from simdonnx_amd.plan import PlanBuilder
+    pb = PlanBuilder()
+    g = offline.graph(pb.build(pb.gemm(pb.input((m, k), None, "a"), np.zeros((k, n), np.float32), None, name="gemm")), storage)
+    kernels = g.kernels
+    g.release()
+    assert len(kernels) == 1, kernels
+    return kernels[0]
+
+
+@pytest.mark.parametrize("storage", STORAGES)
+def test_ragged_rows_take_the_implicit_gemm_where_it_is_faster(offline, storage, monkeypatch):
+    """Products whose rows are not whole 4-element groups: many outputs over a short reduction go to the implicit GEMM
+    (the ring stores them as single elements), few outputs, long reductions and whole groups to the ring."""
+    for shape in ((20000, 16, 1142), (8000, 24, 301), (1500, 40, 5058)):
+        assert "igemm" in _gemm_kernel(offline, storage, *shape), shape
+    for shape in ((20000, 16, 1144), (512, 320, 301), (20000, 768, 301), (4096, 768, 3072), (130, 200, 200)):
+        assert "igemm" not in _gemm_kernel(offline, storage, *shape), shape
+    monkeypatch.setenv("SIMDONNX_HIP_RING", "1")
+    assert "igemm" not in _gemm_kernel(offline, storage, 20000, 16, 1142)
+
+
+def test_fp32_convs_of_few_channels_take_the_implicit_gemm(offline):
+    """fp32 convs over 4 or 8 channels: the implicit GEMM packs their taps where the ring's slices are mostly zeros;
+    from 64 channels on the ring, as do few output tiles from 8 channels on."""
+    for shape in ((1, 128, 277, 4, 366, 5, 1), (1, 20, 20, 4, 8, 3, 1), (4, 250, 16, 8, 344, 3, 1), (1, 223, 150, 8, 408, 2, 1)):
+        assert "igemm" in _conv_kernel(offline, "f32", *shape), shape
+    for shape in ((1, 20, 20, 8, 64, 3, 1), (1, 40, 40, 40, 64, 3, 1), (4, 64, 64, 128, 128, 3, 1), (1, 160, 160, 96, 24, 3, 1)):
+        assert "igemm" not in _conv_kernel(offline, "f32", *shape), shape
