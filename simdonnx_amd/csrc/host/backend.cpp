@@ -884,7 +884,7 @@ struct Emitter {
             {"sox_gemm_f16_128x128_k64s2", 128, 128, 64, 2, 0.72f, 0.67f, 4.0f, 1.6f},
             {"sox_gemm_f16_128x64_k64s2e", 128, 64, 64, 2, 0.46f, 0.345f, 3.9f, 0.4f},
             {"sox_gemm_f16_64x64_k64s2", 64, 64, 64, 4, 0.256f, 0.22f, 3.5f, 0.35f},
-            {"sox_gemm_f16_128x32_k64s2", 128, 32, 64, 3, 0.32f, 0.25f, 2.4f, 0.7f},  // n <= 32
+            {"sox_gemm_f16_128x32_k64s2", 128, 32, 64, 3, 0.32f, 0.25f, 3.2f, 0.7f},  // n <= 32
             // selectable with SIMDONNX_HIP_GEMM (tuning / tests)
             {"sox_gemm_f16_128x64_k64s2", 128, 64, 64, 3},     {"sox_gemm_f16_64x64_k64s4", 64, 64, 64, 2},
             {"sox_gemm_f16_128x64_k64s4", 128, 64, 64, 1},     {"sox_gemm_f16_256x192_k32s5", 256, 192, 32, 1},
@@ -900,7 +900,7 @@ struct Emitter {
             {"sox_gemm_kt_f16_64x64_k64s2", 64, 64, 64, 4, 0.3f, 0.25f, 3.5f, 0.35f},
             {"sox_gemm_kt_f16_128x96_k32s2", 128, 96, 32, 3, 0.3f, 0.26f, 4.0f, 0.7f},
             {"sox_gemm_kt_f16_64x64_k32s2", 64, 64, 32, 4, 0.19f, 0.16f, 3.4f, 0.35f},
-            {"sox_gemm_kt_f16_128x32_k32s2", 128, 32, 32, 4, 0.4f, 0.16f, 2.9f, 0.5f}};  // n <= 32
+            {"sox_gemm_kt_f16_128x32_k32s2", 128, 32, 32, 4, 0.4f, 0.16f, 3.2f, 0.5f}};  // n <= 32
         static const RingCfg cfgs32[] = {
             {"sox_gemm_f32_128x64_k32s2", 128, 64, 32, 3, 1.23f, 1.23f, 4.0f, 1.0f},
             {"sox_gemm_f32_64x64_k32s2", 64, 64, 32, 4, 0.62f, 0.62f, 3.5f, 0.6f},
@@ -909,7 +909,8 @@ struct Emitter {
         const char* forced = getenv("SIMDONNX_HIP_GEMM");
         const RingCfg* pick;
         // a 32-wide 16-bit tile only where every wider one is at least half padding: over more columns it reads
-        // A once more per 32 of them (57600 x 72 -> 40: 6.9 us against 64x64's 5.8)
+        // A once more per 32 of them (57600 x 72 -> 40: 6.9 us against 64x64's 5.8). Its base puts it behind 64x64
+        // for few rows (8 x 24 -> 24 3.3 us on 128x32, 2.7 on 64x64; 57600 x 96 -> 24 4.5 and 5.9)
         const int narrow = a.n <= 32 && !ln ? 1 : 0;
         const bool ragged = ((a.flags & SOX_F_PAD_ROWS) ? a.ldy : a.ldy | a.n) % 4 != 0;
         float est;

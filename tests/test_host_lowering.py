@@ -360,3 +360,13 @@ def test_fp32_convs_of_few_channels_take_the_implicit_gemm(offline):
         assert "igemm" in _conv_kernel(offline, "f32", *shape), shape
     for shape in ((1, 20, 20, 8, 64, 3, 1), (1, 40, 40, 40, 64, 3, 1), (4, 64, 64, 128, 128, 3, 1), (1, 160, 160, 96, 24, 3, 1)):
         assert "igemm" not in _conv_kernel(offline, "f32", *shape), shape
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+def test_narrow_tile_is_for_many_rows(offline, storage):
+    """The 128x32 tile takes products of at most 32 columns over many rows; few rows take 64x64, which costs less."""
+    for k, kt in ((24, f"sox_gemm_kt_{storage}_128x32_k32s2"), (128, f"sox_gemm_{storage}_128x32_k64s2")):
+        for n in (8, 24, 32):
+            assert _gemm_kernel(offline, storage, 66000, k, n) == kt
+            for m in (1, 8, 47):
+                assert "_64x64_" in _gemm_kernel(offline, storage, m, k, n), (m, k, n)
