@@ -2677,8 +2677,7 @@ void fold_layernorm_into_gemm(sox_graph& g) {
         if (xv.count() / K < 64 && fusable_attention(g, gi, x) < 0 && !fusable_mlp(g, gi, x, probe)) continue;
         PlanValue w2 = wv, b2, c2;
         w2.name = wv.name + ".ln";
-        std::vector<double> bsum(N, 0.0), csum(N, 0.0), wsq(N, 0.0), esq(N, 0.0);
-        bool finite = true;
+        std::vector<double> bsum(N, 0.0), csum(N, 0.0);
         for (int k = 0; k < K; k++)
             for (int n = 0; n < N; n++) {
                 const size_t at = gp.trans_b ? (size_t)n * K + k : (size_t)k * N + n;
@@ -2686,23 +2685,26 @@ void fold_layernorm_into_gemm(sox_graph& g) {
                 w2.floats[at] = w * gv.floats[k];
                 bsum[n] += (double)bv.floats[k] * w;
             }
-        std::vector<float> w16(w2.floats.size());
+        std::vector<float> w16(w2.floats.size()), wsq(N, 0.0f), esq(N, 0.0f);
         g.round16(w2.floats.data(), w16.data(), (int64_t)w16.size());
-        for (int k = 0; k < K; k++)
-            for (int n = 0; n < N; n++) {
-                const size_t at = gp.trans_b ? (size_t)n * K + k : (size_t)k * N + n;
-                const double v = w2.floats[at], stored = w16[at];
-                csum[n] += stored;
-                wsq[n] += v * v;
-                if (!g.bf16 && std::fabs(v) < 0x1p-14) esq[n] += (stored - v) * (stored - v);
-                finite = finite && std::isfinite(stored);
+        const float normal = g.bf16 ? 0.0f : 0x1p-14f;
+        for (int i = 0; i < (gp.trans_b ? N : K); i++) {
+            const int len = gp.trans_b ? K : N;
+            const float *v = &w2.floats[(size_t)i * len], *r = &w16[(size_t)i * len];
+            for (int j = 0; j < len; j++) {
+                const int n = gp.trans_b ? i : j;
+                const float lost = std::fabs(v[j]) < normal ? r[j] - v[j] : 0.0f;
+                csum[n] += r[j];
+                wsq[n] += v[j] * v[j];
+                esq[n] += lost * lost;
             }
+        }
         // gamma W has to fit fp16 as W does: finite, and what a column's values below the normal range lose stays
         // under what rounding takes from the others (0.15 of half a unit in the last place, squared). Weights of
         // 0.02 under gamma 1e-3, 16 rows of 192: 9.3e-4 from 64 bits folded, 3.7e-4 as two nodes (gamma 3e-3 4.3e-4 and
         // 3.6e-4, gamma 1e-2 3.6e-4 both, gamma 1 3.0e-4 and 3.7e-4).
-        bool keeps = finite;
-        for (int n = 0; n < N; n++) keeps = keeps && esq[n] <= 0.15 * 0x1p-22 * wsq[n];
+        bool keeps = true;
+        for (int n = 0; n < N; n++) keeps = keeps && std::isfinite(csum[n]) && esq[n] <= 0.15f * 0x1p-22f * wsq[n];
         if (!keeps) continue;
         b2.is_const = c2.is_const = true;
         b2.shape = c2.shape = {N};
