@@ -816,15 +816,16 @@ struct Emitter {
     static float ragged_us(const RingCfg& c, int64_t m, int64_t n) {
         return (c.name == kF32Split ? 0.7e-6f : 2.5e-6f) * (float)(m * n);
     }
-    // The tiling of an m x n product over `taps` taps of k reduction elements each: the forced one, else the
-    // one of [first, last) with the smallest estimate (est, where the caller wants it)
+    // The tiling of an m x n product over `taps` taps of k reduction elements each: the forced one where the table
+    // holds it (where it does not: an error naming `what`, or without `what` no matter), else the one of [first, last)
+    // with the smallest estimate (est)
     const RingCfg& ring_pick(const RingCfg* cfgs, size_t ncfg, int first, int last, int64_t m, int64_t n, int64_t k, int64_t taps,
-                             bool ragged, const char* forced, const char* what, float* est = nullptr) const {
-        if (est) *est = 0.0f;
+                             bool ragged, const char* forced, const char* what, float* est) const {
+        *est = 0.0f;
         if (forced && *forced) {
             for (size_t i = 0; i < ncfg; i++)
                 if (!strcmp(cfgs[i].name, forced)) return cfgs[i];
-            fail(SOX_E_INVALID, std::string(what) + ": unknown kernel " + forced);
+            if (what) fail(SOX_E_INVALID, std::string(what) + ": unknown kernel " + forced);
         }
         const int64_t cus = std::max(1, g.be->info.compute_units);
         int pick = first;
@@ -838,7 +839,7 @@ struct Emitter {
                 best = t;
             }
         }
-        if (est) *est = best;
+        *est = best;
         return cfgs[pick];
     }
 
@@ -914,8 +915,8 @@ struct Emitter {
         const int narrow = a.n <= 32 && !ln ? 1 : 0;
         const bool ragged = ((a.flags & SOX_F_PAD_ROWS) ? a.ldy : a.ldy | a.n) % 4 != 0;
         float est;
-        if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, ragged, nullptr, "", &est);
-        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 7, 0, 6 + narrow, a.m, a.n, a.k, 1, ragged, nullptr, "", &est);
+        if (!g.f16) pick = &ring_pick(cfgs32, 4, 0, 4, a.m, a.n, a.k, 1, ragged, forced, nullptr, &est);
+        else if (a.k % 64 != 0) pick = &ring_pick(cfgs_kt, 7, 0, 6 + narrow, a.m, a.n, a.k, 1, ragged, forced, nullptr, &est);
         else pick = &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), ln ? 1 : 0, 5 + narrow, a.m, a.n, a.k, 1, ragged, forced, "SIMDONNX_HIP_GEMM", &est);
         if (igemm && igemm_wins(est, a.m, a.n, a.k, igemm, ragged)) {
             if (igemm == 'd') {
@@ -1014,10 +1015,11 @@ struct Emitter {
             name = "sox_conv_f16_256x128_w8k64s2";
         const int64_t taps = (int64_t)a.kh * a.kw;
         const bool ragged = !(a.flags & SOX_F_CONVT) && (a.ldy | a.n) % 4 != 0;
+        const int ncfg32 = a.flags & SOX_F_REFLECT ? 3 : 4;
         float est = 0.0f;
         const RingCfg* c =
-            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 8 : 7, a.m, a.n, a.ic, taps, ragged, name, "SIMDONNX_HIP_CONV")
-                  : &ring_pick(cfgs32, 4, 0, a.flags & SOX_F_REFLECT ? 3 : 4, a.m, a.n, a.ic, taps, ragged, nullptr, "", &est);
+            g.f16 ? &ring_pick(cfgs16, sizeof(cfgs16) / sizeof(cfgs16[0]), 0, a.n <= 32 ? 8 : 7, a.m, a.n, a.ic, taps, ragged, name, "SIMDONNX_HIP_CONV", &est)
+                  : &ring_pick(cfgs32, ncfg32, 0, ncfg32, a.m, a.n, a.ic, taps, ragged, name, nullptr, &est);
         if (!g.f16 && igemm_wins(est, a.m, a.n, a.k, 'v', ragged)) {
             launch_igemm(node, a, x, w, bias, add_b, y, 'v', "conv");
             return;

@@ -370,3 +370,33 @@ def test_narrow_tile_is_for_many_rows(offline, storage):
             assert _gemm_kernel(offline, storage, 66000, k, n) == kt
             for m in (1, 8, 47):
                 assert "_64x64_" in _gemm_kernel(offline, storage, m, k, n), (m, k, n)
+
+
+# a shape that takes each tiling by the estimate, at 256 CUs: (rows, k, n), or (batch, h, w, channels, oc, kernel, stride)
+TILING_SHAPES = {
+    "sox_gemm_f16_256x192_w8k64s2": (8192, 768, 3072), "sox_gemm_f16_256x128_w8k64s2": (21124, 64, 280),
+    "sox_gemm_f16_128x128_k64s2": (19893, 3072, 1352), "sox_gemm_f16_128x64_k64s2e": (25612, 64, 68),
+    "sox_gemm_f16_64x64_k64s2": (1, 64, 15), "sox_gemm_f16_128x32_k64s2": (18889, 128, 10),
+    "sox_gemm_kt_f16_256x128_w8k64s2": (3769, 8, 1988), "sox_gemm_kt_f16_128x128_k64s2": (1264, 408, 3042),
+    "sox_gemm_kt_f16_128x64_k64s2": (19563, 136, 296), "sox_gemm_kt_f16_64x64_k64s2": (2, 232, 9),
+    "sox_gemm_kt_f16_128x96_k32s2": (6202, 8, 908), "sox_gemm_kt_f16_64x64_k32s2": (1, 8, 8),
+    "sox_gemm_kt_f16_128x32_k32s2": (23362, 8, 12), "sox_gemm_f32_128x64_k32s2": (8192, 512, 1024),
+    "sox_gemm_f32_64x64_k32s2": (786, 760, 760), "sox_gemm_f32_128x32_k32s2": (12300, 40, 192),
+    "sox_conv_f32_split": (40, 192, 768), "sox_conv_f16_128x128_k64s2": (8, 64, 64, 128, 256, 3, 1),
+    "sox_conv_f16_128x128_k32s4": (8, 93, 91, 24, 112, 5, 1), "sox_conv_f16_128x96_k64s2": (2, 160, 160, 40, 80, 3, 1),
+    "sox_conv_f16_128x96_k32s2": (2, 95, 127, 96, 168, 3, 1), "sox_conv_f16_128x64_k64s2": (1, 184, 190, 40, 35, 3, 1),
+    "sox_conv_f16_64x64_k64s4": (1, 6, 4, 48, 15, 3, 2), "sox_conv_f16_64x64_k32s4": (1, 5, 5, 8, 15, 3, 1),
+    "sox_conv_f16_128x32_k32s2": (4, 47, 137, 8, 9, 3, 1), "sox_conv_f32_128x64_k32s2": (8, 35, 54, 56, 223, 3, 1),
+    "sox_conv_f32_64x64_k32s4": (4, 6, 100, 24, 268, 3, 1), "sox_conv_f32_128x32_k32s2": (2, 147, 96, 32, 9, 3, 1)}
+
+
+def test_every_tiling_of_the_estimate_is_taken_by_some_shape(offline, monkeypatch):
+    """No table entry is out of the estimate's reach, and the numeric tests' list of tilings (test_gpu_ring.tilings, read
+    from the tables) is the list of these shapes."""
+    from tests.test_gpu_ring import tilings
+    assert {n.split()[0] for _, n in tilings()} == set(TILING_SHAPES)
+    monkeypatch.setenv("SIMDONNX_HIP_NOHALO", "1")
+    for name, shape in TILING_SHAPES.items():
+        for storage in ("f32",) if "_f32_" in name else ("f16", "bf16"):
+            got = _gemm_kernel(offline, storage, *shape) if len(shape) == 3 else _conv_kernel(offline, storage, *shape)
+            assert got == name.replace("_f16_", f"_{storage}_"), (name, shape, got)
