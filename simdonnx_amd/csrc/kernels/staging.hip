@@ -8,8 +8,9 @@
 //   in  (fp32 -> fp16):  1.0 MB 36.7 / 31.5 us,  5.9 MB 123 / 118 us,  11.1 MB 215 / 209 us,  30 MB 551 / 540 us
 //   out (fp16 -> fp32):  1.0 MB 38.7 / 29.0 us,  5.9 MB 132 / 117 us,  11.1 MB 223 / 210 us,  30 MB 557 / 556 us
 // Reading host memory wants few requests in flight over few distinct pages: 64 workgroups with two 16-byte
-// loads per thread in flight (128 KiB) come within 5% of the copy engine at every size, 256 workgroups with
-// eight take 245 us for the 11.1 MB. Writes are posted: 256 workgroups with four stores each.
+// loads per thread in flight (512 KiB) keep up with the copy engine at every size (a whole call with 64 / 256 /
+// 512 MB going up: engine + conversion 1234 / 4847 / 9660 us, here 1207 / 4762 / 9505; fp32 1234 / 4829 / 9627 and 1214 /
+// 4783 / 9597), 256 workgroups with eight take 245 us for the 11.1 MB. Writes are posted: 256 workgroups with four stores each.
 #include "sox_device.h"
 
 namespace {
