@@ -88,8 +88,8 @@ SOX_DEV float sox_act(float v, int act) {
 // L is the least-squares fit of log2(1 - Phi(a)) on [0, 5.5], reweighted toward the minimax error
 // (max |error of L| 3.7e-5). Against the exact erf-GELU in float64 its float32 evaluation is off by at
 // most 3.9e-6 absolute and 2.7e-5 relative (|gelu| >= 1e-3): every fp16 value in [-8, 8] rounds to
-// within 0.55 ulp of the exact GELU, every bf16 value to within 0.51 ulp. The clamp and the ReLU are
-// one v_med3_f32 each (no canonicalising max). Cost: 10 full-rate instructions and one exp2, against
+// within 0.55 ulp of the exact GELU, every bf16 value to within 0.51 ulp. The clamp is one v_med3_f32, the
+// ReLU one v_maximum3_f32, which keeps a NaN (v_max_f32 and v_med3_f32 drop it: gelu(NaN) would be 0). Cost: 10 full-rate instructions and one exp2, against
 // 15 and an exp2 plus a reciprocal for the A&S form of sox_gelu (v_rcp_f32 / v_exp_f32 issue at a
 // quarter of the rate).
 // In two halves of about five instructions each (gelu_fast_lo: the clamp and the polynomial's first
@@ -106,7 +106,7 @@ SOX_DEV float gelu_fast_hi(float x, float a, float l) {
     l = __builtin_fmaf(l, a, -0.4603187143802643f);
     l = __builtin_fmaf(l, a, -1.150593876838684f);
     l = __builtin_fmaf(l, a, -1.000033974647522f);
-    return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(l), __builtin_amdgcn_fmed3f(x, 0.0f, __builtin_inff()));
+    return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(l), __builtin_elementwise_maximum(x, 0.0f));
 }
 SOX_DEV float gelu_fast(float x) {
     float a, l;

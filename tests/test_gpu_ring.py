@@ -318,3 +318,39 @@ def test_fp32_convs_on_the_implicit_gemm(hip, case, monkeypatch):
     want = O.conv(x, wt, b, r, stride=(st, st), pads=(p, p, p, p), act=act, pad_mode=mode, algo=1)
     if cat: want = np.concatenate([O.conv(x, wt[:8], b[:8], stride=(1, 1), pads=(1, 1, 1, 1), act="none", algo=1), want], axis=-1)
     assert max_rel(got, want) < tol("f32", k * k * ic), kernels
+
+
+NAN_GEMMS = [(5, 8, 24), (33, 40, 104), (7, 96, 219), (951, 248, 93), (300, 128, 200), (4, 39, 154), (4100, 192, 776), (16400, 64, 24)]
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16", "f32"])
+def test_gelu_keeps_nan(hip, storage, monkeypatch):
+    """A NaN reaches the outputs that depend on it, and only those, through every kernel's GELU: dense products, convs
+    (ring, halo) and the MLP of few and many rows."""
+    for m, k, n in NAN_GEMMS:
+        x = stored(synth.normal(151, 1, (m, k), 1.0), storage)
+        x[m // 2, k // 3] = np.nan
+        pb = PlanBuilder()
+        y = pb.gemm(pb.input((m, k), None, "x"), synth.normal(151, 2, (k, n), k**-0.5), None, act="gelu", name="gemm")
+        got, kernels = run(hip, pb.build(y), [x], storage)
+        nan = np.isnan(got.reshape(m, n))
+        assert nan[m // 2].all() and nan.sum() == n, (m, k, n, kernels)
+    for h, w, ic, oc, k in ((19, 33, 24, 40, 3), (40, 50, 96, 100, 3), (30, 30, 64, 256, 3), (21, 20, 16, 72, 1), (20, 20, 16, 24, 5)):
+        x = synth.normal(151, 3, (1, h, w, ic), 1.0)
+        x[0, 9, 11, ic // 2] = np.nan
+        wt = synth.normal(151, 4, (oc, ic, k, k), (k * k * ic)**-0.5)
+        for nohalo in (False, True):
+            monkeypatch.setenv("SIMDONNX_HIP_NOHALO", "1") if nohalo else monkeypatch.delenv("SIMDONNX_HIP_NOHALO", raising=False)
+            pb = PlanBuilder()
+            y = pb.conv(pb.input((1, ic, h, w), NHWC, "x"), wt, None, pad=k // 2, act="gelu", name="conv")
+            got, kernels = run(hip, pb.build(y), [x], storage)
+            assert np.array_equal(np.isnan(got), np.isnan(O.conv(x, wt, None, pads=(k // 2,) * 4, act="gelu", algo=1))), kernels
+    for rows in (3, 63, 200):
+        x = synth.normal(151, 5, (1, rows, 192), 1.0)
+        x[0, rows // 2, 7] = np.nan
+        pb = PlanBuilder()
+        h = pb.layer_norm(pb.input((1, rows, 192), None, "x"), np.ones(192, np.float32), np.zeros(192, np.float32), 1e-6, name="ln")
+        h = pb.gemm(h, synth.normal(151, 6, (192, 768), 0.05), np.zeros(768, np.float32), act="gelu", name="fc1")
+        got, kernels = run(hip, pb.build(pb.gemm(h, synth.normal(151, 7, (768, 192), 0.05), np.zeros(192, np.float32), name="fc2")), [x], storage)
+        nan = np.isnan(got.reshape(rows, 192))
+        assert nan[rows // 2].all() and nan.sum() == 192, (rows, kernels)
